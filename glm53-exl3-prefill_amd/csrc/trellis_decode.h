@@ -7,18 +7,21 @@
 // A lane decodes one chunk: the 8 positions p = 8c + j (c = chunk 0..31, j = 0..7), which sit at tile rows
 // k = 2(c & 3) + (j & 1) + 8((j >> 1) & 1) and columns n = (c >> 2) + 8(j >> 2).
 //
-// gfx950 cost per weight: the 32-bit multiply by a 16-bit state is split into a 16x16 low-half multiply whose
-// result lands in the upper word (SDWA) plus a 16x16+32 multiply-add that picks the state's half by op_sel,
-// so no state ever needs shifting out of its dword; v_bitop3 does mask-and-xor in one op, and SDWA fp16 adds write
-// each sum into its half of the packed output pair in place. About 4.4 VALU ops per weight at 4 bits.
+// gfx950 cost per weight. Measured per wave64 instruction and SIMD at four waves per SIMD (2.1-2.4 GHz): v_mul_lo_u32,
+// v_mad_u32_u16, v_bfe_u32, v_alignbit_b32 and every SDWA form 2.4 cycles; right shifts, v_and_b32 and v_bitop3_b32
+// 1.6-1.7. A full 32-bit product thus costs no more than either half of a product built from 16-bit multiplies, so a
+// state is cut out of its dwords by one v_bfe_u32 (a right shift where it is the upper half) and multiplied by one
+// v_mul_lo_u32; v_bitop3 does mask-and-xor in one op, and SDWA fp16 adds write each sum into its half of the packed
+// output pair in place. About 4.1 VALU ops per weight. A register-only loop of this decode and two MFMAs per 16 weights
+// runs 12.3 T weights/s on the device at four waves per SIMD (2.28 GHz), against 10.7 (2.20 GHz) with the product as
+// an SDWA 16-bit multiply into the upper word and a v_mad_u32_u16.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 namespace exl3 {
 
-constexpr uint32_t MCG_MUL_LO = 0x1FEDu;       // low 16 bits of 0xCBAC1FED
-constexpr uint32_t MCG_MUL_HI = 0xCBACu;       // high 16 bits
+constexpr uint32_t MCG_MUL = 0xCBAC1FEDu;
 constexpr uint32_t MCG_XOR = 0x3B603B60u;
 constexpr uint32_t MCG_MASK = 0x8FFF8FFFu;
 
@@ -30,39 +33,25 @@ constexpr uint32_t MCG_MASK = 0x8FFF8FFFu;
 // from instructions with wait-state rules of their own (per-lane 64-bit shifts fed into them gave wrong results at
 // random): callers hand them 32-bit funnel shifts, loads and DPP moves.
 
-// x0 = (SEL0 ? hi : lo)(ra) * 0xCBAC1FED, x1 = (SEL1 ? hi : lo)(rb) * 0xCBAC1FED  (mod 2^32), as full 32-bit products.
-#define EXL3_MCG_MUL2(S0, S1, OP0, OP1)                                                                               \
-    asm("v_mul_lo_u16_sdwa %0, %4, %6 dst_sel:WORD_1 dst_unused:UNUSED_PAD src0_sel:" S0 " src1_sel:DWORD\n\t"       \
-        "v_mul_lo_u16_sdwa %1, %5, %6 dst_sel:WORD_1 dst_unused:UNUSED_PAD src0_sel:" S1 " src1_sel:DWORD\n\t"       \
-        "v_mad_u32_u16 %2, %4, %7, %0" OP0 "\n\t"                                                                    \
-        "v_mad_u32_u16 %3, %5, %7, %1" OP1                                                                          \
-        : "=&v"(t0), "=&v"(t1), "=&v"(x0), "=&v"(x1) : "v"(ra), "v"(rb), "s"(chi), "s"(clo))
-template <int SEL0, int SEL1>
-__device__ __forceinline__ void mcg_mul2(uint32_t ra, uint32_t rb, uint32_t& x0, uint32_t& x1)
-{
-    uint32_t t0, t1;
-    const uint32_t chi = MCG_MUL_HI, clo = MCG_MUL_LO;
-    if constexpr (!SEL0 && !SEL1) EXL3_MCG_MUL2("WORD_0", "WORD_0", "", "");
-    else if constexpr (!SEL0 && SEL1) EXL3_MCG_MUL2("WORD_0", "WORD_1", "", " op_sel:[1,0,0,0]");
-    else if constexpr (SEL0 && !SEL1) EXL3_MCG_MUL2("WORD_1", "WORD_0", " op_sel:[1,0,0,0]", "");
-    else EXL3_MCG_MUL2("WORD_1", "WORD_1", " op_sel:[1,0,0,0]", " op_sel:[1,0,0,0]");
-}
-#undef EXL3_MCG_MUL2
+// The code's two fp16 halves of a state isolated in the low 16 bits.
+__device__ __forceinline__ uint32_t mcg_halves(uint32_t state) { return ((state * MCG_MUL) & MCG_MASK) ^ MCG_XOR; }
 
-__device__ __forceinline__ uint32_t mcg_mask(uint32_t x) { return (x & MCG_MASK) ^ MCG_XOR; }
-
-// Two packed fp16 pairs: w0 = {fp16(ya.lo + ya.hi), fp16(yb.lo + yb.hi)}, w1 = {same for yc, yd}. The low halves are
-// written first (upper half zeroed), then the high halves with the low ones preserved -- each read-modify-write two
-// instructions after the write it reads -- and an s_nop guards the last partial write.
-__device__ __forceinline__ void add_halves_2pairs(uint32_t ya, uint32_t yb, uint32_t yc, uint32_t yd,
-                                                  uint32_t& w0, uint32_t& w1)
+// Four packed fp16 pairs from eight codes' halves: w[i] = {fp16(y[2i].lo + y[2i].hi), fp16(y[2i+1].lo + y[2i+1].hi)}.
+// The low halves are written first (upper half zeroed), then the high halves with the low ones preserved -- each
+// read-modify-write four instructions after the write it reads -- and an s_nop guards the last partial write.
+__device__ __forceinline__ void add_halves_4pairs(const uint32_t (&y)[8], uint32_t (&w)[4])
 {
-    asm("v_add_f16_sdwa %0, %2, %2 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
-        "v_add_f16_sdwa %1, %4, %4 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
-        "v_add_f16_sdwa %0, %3, %3 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
-        "v_add_f16_sdwa %1, %5, %5 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+    asm("v_add_f16_sdwa %0, %4, %4 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+        "v_add_f16_sdwa %1, %6, %6 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+        "v_add_f16_sdwa %2, %8, %8 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+        "v_add_f16_sdwa %3, %10, %10 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+        "v_add_f16_sdwa %0, %5, %5 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+        "v_add_f16_sdwa %1, %7, %7 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+        "v_add_f16_sdwa %2, %9, %9 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+        "v_add_f16_sdwa %3, %11, %11 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
         "s_nop 1"
-        : "=&v"(w0), "=&v"(w1) : "v"(ya), "v"(yb), "v"(yc), "v"(yd));
+        : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3])
+        : "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(y[4]), "v"(y[5]), "v"(y[6]), "v"(y[7]));
 }
 
 // Decoded chunk, as four packed fp16 pairs ordered for a [n][k] (k-contiguous) destination:
@@ -70,65 +59,44 @@ __device__ __forceinline__ void add_halves_2pairs(uint32_t ya, uint32_t yb, uint
 //   out[3] = (k0+8, k0+9) at n0+8, with k0 = 2(c & 3), n0 = c >> 2.
 struct Chunk4 { uint32_t w[4]; };
 
-// Per-lane constants locating chunk c's bits: the two dwords (lo, hi) holding them and the bit offset of the
-// window of position 8c inside the 64-bit value hi:lo.
-struct ChunkLoc { int dlo, dhi, off; };
-
-template <int BITS>
-__device__ __forceinline__ ChunkLoc chunk_loc(int c)
+// The 16-bit state starting OFF bits into hi:lo, from lo, hi or the dword across them (mid = bits 16 .. 47).
+template <int OFF>
+__device__ __forceinline__ uint32_t state_at(uint32_t lo, uint32_t mid, uint32_t hi)
 {
-    constexpr int NDW = 8 * BITS;                          // dwords per tile
-    const int b0 = 8 * c * BITS + BITS - 16;               // first stream bit of position 8c's window
-    const int d0 = (b0 >= 0) ? (b0 >> 5) : -1;            // floor(b0 / 32), b0 >= -15
-    ChunkLoc L;
-    L.off = b0 - 32 * d0;
-    L.dlo = (d0 + NDW) % NDW;
-    L.dhi = (d0 + 1) % NDW;
-    return L;
+    static_assert(OFF >= 0 && OFF <= 48, "a state within 64 bits");
+    if constexpr (OFF <= 16) return (lo >> OFF) & 0xFFFF;
+    else if constexpr (OFF <= 32) return (mid >> (OFF - 16)) & 0xFFFF;
+    else return (hi >> (OFF - 32)) & 0xFFFF;
 }
 
-// Decode the chunk whose stream bits sit in hi:lo starting at bit `off` (BITS in {1,2,3,4}).
-template <int BITS>
-__device__ __forceinline__ Chunk4 decode_chunk(uint32_t lo, uint32_t hi, int off)
+// Decode the chunk whose stream bits sit in hi:lo starting at bit OFF (BITS in {1,2,3,4}).
+template <int BITS, int OFF>
+__device__ __forceinline__ Chunk4 decode_chunk(uint32_t lo, uint32_t hi)
 {
-    uint32_t x[8];
-    if constexpr (BITS == 4)
-    {
-        // off == 20 for every chunk: states j and j+4 are the low/high halves of one shifted dword
-        const uint32_t r0 = hi;                                      // states 3, 7
-        const uint32_t r1 = __builtin_amdgcn_alignbit(hi, lo, 20);   // states 0, 4
-        const uint32_t r2 = __builtin_amdgcn_alignbit(hi, lo, 24);   // states 1, 5
-        const uint32_t r3 = __builtin_amdgcn_alignbit(hi, lo, 28);   // states 2, 6
-        mcg_mul2<0, 1>(r1, r1, x[0], x[4]);
-        mcg_mul2<0, 1>(r2, r2, x[1], x[5]);
-        mcg_mul2<0, 1>(r3, r3, x[2], x[6]);
-        mcg_mul2<0, 1>(r0, r0, x[3], x[7]);
-    }
-    else
-    {
-        const uint64_t q = ((uint64_t) hi << 32) | lo;
-        uint32_t r[8];
-        #pragma unroll
-        for (int j = 0; j < 8; ++j) r[j] = (uint32_t) (q >> (off + j * BITS));
-        #pragma unroll
-        for (int j = 0; j < 8; j += 2) mcg_mul2<0, 0>(r[j], r[j + 1], x[j], x[j + 1]);
-    }
-    uint32_t y[8];
-    #pragma unroll
-    for (int j = 0; j < 8; ++j) y[j] = mcg_mask(x[j]);
+    const uint32_t mid = __builtin_amdgcn_alignbit(hi, lo, 16);
+    const uint32_t y[8] = {mcg_halves(state_at<OFF>(lo, mid, hi)), mcg_halves(state_at<OFF + BITS>(lo, mid, hi)),
+                           mcg_halves(state_at<OFF + 2 * BITS>(lo, mid, hi)),
+                           mcg_halves(state_at<OFF + 3 * BITS>(lo, mid, hi)),
+                           mcg_halves(state_at<OFF + 4 * BITS>(lo, mid, hi)),
+                           mcg_halves(state_at<OFF + 5 * BITS>(lo, mid, hi)),
+                           mcg_halves(state_at<OFF + 6 * BITS>(lo, mid, hi)),
+                           mcg_halves(state_at<OFF + 7 * BITS>(lo, mid, hi))};
     Chunk4 c;
-    add_halves_2pairs(y[0], y[1], y[2], y[3], c.w[0], c.w[1]);
-    add_halves_2pairs(y[4], y[5], y[6], y[7], c.w[2], c.w[3]);
+    add_halves_4pairs(y, c.w);
     return c;
 }
 
-// Decode four independent states (low and high halves of ra and rb) -> packed fp16 pairs (wa for ra, wb for rb).
-__device__ __forceinline__ void decode_state_pairs(uint32_t ra, uint32_t rb, uint32_t& wa, uint32_t& wb)
+// Decode four dwords of two independent states each -> packed fp16 pairs, one dword per input dword.
+__device__ __forceinline__ void decode_states_4(const uint32_t (&r)[4], uint32_t (&w)[4])
 {
-    uint32_t x0, x1, x2, x3;
-    mcg_mul2<0, 1>(ra, ra, x0, x1);
-    mcg_mul2<0, 1>(rb, rb, x2, x3);
-    add_halves_2pairs(mcg_mask(x0), mcg_mask(x1), mcg_mask(x2), mcg_mask(x3), wa, wb);
+    uint32_t y[8];
+    #pragma unroll
+    for (int i = 0; i < 4; ++i)
+    {
+        y[2 * i] = mcg_halves(r[i] & 0xFFFF);
+        y[2 * i + 1] = mcg_halves(r[i] >> 16);
+    }
+    add_halves_4pairs(y, w);
 }
 
 }  // namespace exl3

@@ -298,14 +298,14 @@ struct Decoder
         if constexpr (BITS == 4)
         {
             const uint32_t prev = prev_in_row(r[1]);
-            c0 = decode_chunk<4>(prev, r[0], 20);
-            c1 = decode_chunk<4>(r[0], r[1], 20);
+            c0 = decode_chunk<4, 20>(prev, r[0]);
+            c1 = decode_chunk<4, 20>(r[0], r[1]);
         }
         else if constexpr (BITS == 2)
         {
             const uint32_t prev = prev_in_row(r[0]);
-            c0 = decode_chunk<2>(prev, r[0], 18);
-            c1 = decode_chunk<2>(r[0], r[0], 2);              // window ends inside r[0]
+            c0 = decode_chunk<2, 18>(prev, r[0]);
+            c1 = decode_chunk<2, 2>(r[0], r[0]);              // window ends inside r[0]
         }
         else
         {
@@ -315,8 +315,8 @@ struct Decoder
             // feeding the decoder's asm gave wrong results at random.
             const uint32_t x0 = tb ? r[0] : __builtin_amdgcn_alignbit(r[1], r[0], 16);
             const uint32_t x1 = tb ? r[1] : __builtin_amdgcn_alignbit(r[2], r[1], 16);
-            c0 = decode_chunk<3>(x0, x1, 3);
-            c1 = decode_chunk<3>(x0, x1, 27);
+            c0 = decode_chunk<3, 3>(x0, x1);
+            c1 = decode_chunk<3, 27>(x0, x1);
         }
     }
     __device__ __forceinline__ void store(const Out& o, uint16_t* lds) const
@@ -371,14 +371,14 @@ struct Decoder1
     __device__ __forceinline__ void decode(const uint32_t (&r)[NR], Out& o) const
     {
         if constexpr (BITS == 4)
-            o.c[0] = decode_chunk<4>(r[0], r[1], 20);             // shift is 20 for every chunk
+            o.c[0] = decode_chunk<4, 20>(r[0], r[1]);             // shift is 20 for every chunk
         else
         {
             // Realign with 32-bit funnel shifts (per-lane 64-bit shift amounts feeding the decoder's asm gave wrong
             // results at random), then decode at the compile-time offset 0.
             const uint32_t x0 = __builtin_amdgcn_alignbit(r[1], r[0], shift);
             const uint32_t x1 = r[1] >> shift;
-            o.c[0] = decode_chunk<BITS>(x0, x1, 0);
+            o.c[0] = decode_chunk<BITS, 0>(x0, x1);
         }
     }
     __device__ __forceinline__ void store(const Out& o, uint16_t* lds) const

@@ -146,13 +146,12 @@ void reconstruct_kernel(uint16_t* __restrict__ out, const uint32_t* __restrict__
     for (int i = 0; i <= BITS; ++i) r[i] = t[(BITS * j - 1 + i + NDW) % NDW];
     const int tk = (int) (tile / tiles_n), tn = (int) (tile % tiles_n);
     const int64_t ncols = (int64_t) tiles_n * 16;
-    #pragma unroll
-    for (int i = 0; i < 4; ++i)
-    {
-        const int b0 = 8 * i * BITS + BITS - 16;
-        const int rel = (b0 >= 0 ? b0 / 32 : -1) + 1;
-        const int off = b0 - 32 * (rel - 1);
-        const Chunk4 c = decode_chunk<BITS>(r[rel], r[rel + 1 <= BITS ? rel + 1 : BITS], off);
+    static_for<4>([&](auto i_tag) {
+        constexpr int i = decltype(i_tag)::value;
+        constexpr int b0 = 8 * i * BITS + BITS - 16;
+        constexpr int rel = (b0 >= 0 ? b0 / 32 : -1) + 1;
+        constexpr int off = b0 - 32 * (rel - 1);
+        const Chunk4 c = decode_chunk<BITS, off>(r[rel], r[rel + 1 <= BITS ? rel + 1 : BITS]);
         // chunk 4j+i: k0 = 2i, columns j and j+8
         #pragma unroll
         for (int q = 0; q < 4; ++q)
@@ -163,19 +162,20 @@ void reconstruct_kernel(uint16_t* __restrict__ out, const uint32_t* __restrict__
             o[0] = (uint16_t) (c.w[q] & 0xFFFF);
             o[ncols] = (uint16_t) (c.w[q] >> 16);
         }
-    }
+    });
 }
 
-// Each thread decodes two dwords (four states); n2 = number of dwords.
+// Each thread decodes four dwords (eight states); n2 = number of dwords.
 __global__ void decode_states_kernel(const uint32_t* __restrict__ states, uint32_t* __restrict__ out, int64_t n2)
 {
-    const int64_t i = 2 * ((int64_t) blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= n2) return;
-    const uint32_t ra = states[i], rb = (i + 1 < n2) ? states[i + 1] : 0u;
-    uint32_t wa, wb;
-    decode_state_pairs(ra, rb, wa, wb);
-    out[i] = wa;
-    if (i + 1 < n2) out[i + 1] = wb;
+    const int64_t i0 = 4 * ((int64_t) blockIdx.x * blockDim.x + threadIdx.x);
+    uint32_t r[4], w[4];
+    #pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = i0 + i < n2 ? states[i0 + i] : 0u;
+    decode_states_4(r, w);
+    #pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (i0 + i < n2) out[i0 + i] = w[i];
 }
 
 template <int MODE, bool DENSE>
@@ -690,7 +690,7 @@ extern "C" int exl3_decode_states(const uint16_t* states, uint16_t* out, int64_t
                "states/out must be 4-byte aligned");
     const int64_t n2 = n / 2;
     if (n2 == 0) return EXL3_OK;
-    decode_states_kernel<<<(unsigned) ((n2 + 511) / 512), 256, 0, as_stream(stream)>>>(
+    decode_states_kernel<<<(unsigned) ((n2 + 1023) / 1024), 256, 0, as_stream(stream)>>>(
         reinterpret_cast<const uint32_t*>(states), reinterpret_cast<uint32_t*>(out), n2);
     return hip_status("decode_states");
 }
