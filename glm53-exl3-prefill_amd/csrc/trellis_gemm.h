@@ -14,7 +14,7 @@
 //     MFMAs run; write stage s+1 into the other LDS buffer; issue loads for later stages. Raw trellis words are
 //     prefetched RAW_DEPTH stages ahead and activations ACT_DEPTH stages ahead, straight into VGPRs. One barrier per
 //     stage guards the double-buffered decoded tile.
-//   * A wave with <= 16 valid rows multiplies one 16-row group, a wave with none only decodes (thin experts).
+//   * A wave with <= 16 valid rows multiplies one 16-row group, a wave with none only decodes.
 //   * Epilogue: H128 with 5 butterfly stages in registers and 2 across lanes, x svh / sqrt(128), fp16 store, fp32
 //     store, fp32 per-route store, or fp32 atomics staged through LDS so each atomic instruction covers 64 consecutive
 //     floats of one output row.
@@ -23,8 +23,9 @@
 //     (row tile, 128-column block) pair of gate and up computes that block of the activation (act_had) itself.
 //   * Activations and trellis words are read through buffer resources: fixed per-lane offsets plus a scalar stage
 //     offset, and zero instead of a fault outside the operand.
-// Variants of the same kernel: 16 rows per wave (64-row tiles, four workgroups per CU) for small tiles, and 8 waves
-// (512-row tiles, one workgroup per CU, each wave decoding one chunk per lane) for 512-row tiles and large dense GEMMs.
+// Variants of the same kernel: 8 waves (512-row tiles, one workgroup per CU, each wave decoding one chunk per lane) for
+// 512-row tiles and large dense GEMMs. 64-row tiles (small batches, each expert's small last tile) run a kernel of their
+// own (thin_tile): four workgroups per CU, each wave decoding its own 32 columns straight into MFMA operands.
 #pragma once
 #include "exl3_common.h"
 #include "hadamard.h"
@@ -53,6 +54,10 @@ constexpr int LDS_BLK = 16 * LDS_ROW + EXL3_LDS_BLK_PAD;   // halves per 16-row 
 constexpr int LDS_TILE = 8 * LDS_BLK;               // halves per decoded stage (128 n-rows)
 constexpr int SC_ROW = TILE_N + 4;                  // floats per staged output row of the scatter epilogue
 constexpr int LDS_MAIN_BYTES = 2 * LDS_TILE * 2;
+constexpr int THIN_CHUNK = 4;                       // 64-row tiles: stages per activation chunk, one per wave
+constexpr int THIN_DEPTH = THIN_CHUNK;              // trellis stages in flight
+constexpr int THIN_LDS_BYTES = 4 * 8 * 64 * 16;     // 64-row tiles: two chunks of four stages x four row groups, then
+                                                    // four row groups' accumulators over 128 columns
 #ifndef EXL3_RAW_DEPTH
 #define EXL3_RAW_DEPTH 4
 #endif
@@ -232,12 +237,37 @@ __device__ __forceinline__ bool resolve_tile(const GemmParams& p, int group, int
 // a = j16 >> 1 and a + 8, rows 4 b .. 4 b + 3 and 8 + 4 b .. with b = j16 & 1.
 template <int N> struct Chunks { Chunk4 c[N]; };
 
-// NT: the raw words are loaded non-temporal (64-row tiles that read each weight once: the prefill's thin launches and
-// the decode path).
-template <int BITS, bool NT = false>
+// Chunks 2 j and 2 j + 1 of a tile (positions 16 j .. + 15): from the tile's dwords 2 j, 2 j + 1 (4 bits) or dword j (2
+// bits) in r with the dword before them in prev, or from the three dwords the two windows touch (3 bits; odd = j & 1).
+template <int BITS>
+__device__ __forceinline__ void decode_pair(uint32_t prev, const uint32_t (&r)[raw_words<BITS>()], int odd, Chunks<2>& o)
+{
+    if constexpr (BITS == 4)
+    {
+        o.c[0] = decode_chunk<4, 20>(prev, r[0]);
+        o.c[1] = decode_chunk<4, 20>(r[0], r[1]);
+    }
+    else if constexpr (BITS == 2)
+    {
+        o.c[0] = decode_chunk<2, 18>(prev, r[0]);
+        o.c[1] = decode_chunk<2, 2>(r[0], r[0]);              // window ends inside r[0]
+    }
+    else
+    {
+        // The windows start 19 / 43 bits (j even) or 3 / 27 bits (odd) into r[0]. Even ones shift their words down by
+        // 16 bits first, so both kinds decode at the compile-time offsets 3 and 27: constant shifts of a 64-bit window
+        // compile to 32-bit funnel shifts, while per-lane 64-bit shift amounts feeding the decoder's asm gave wrong
+        // results at random.
+        const uint32_t x0 = odd ? r[0] : __builtin_amdgcn_alignbit(r[1], r[0], 16);
+        const uint32_t x1 = odd ? r[1] : __builtin_amdgcn_alignbit(r[2], r[1], 16);
+        o.c[0] = decode_chunk<3, 3>(x0, x1);
+        o.c[1] = decode_chunk<3, 27>(x0, x1);
+    }
+}
+
+template <int BITS>
 struct Decoder
 {
-    static constexpr int AUX = NT ? 2 : 0;                // buffer-load cache policy: 2 = non-temporal
     static constexpr int NDW = 8 * BITS;                  // dwords per tile
     static constexpr int NR = raw_words<BITS>();
     using Out = Chunks<2>;
@@ -245,22 +275,18 @@ struct Decoder
     int stage_bytes, last_kb, tb, wcol0, wcol1;
     uint32_t off[NR];              // per-lane byte offsets of the raw words
 
-    // cols: the thin tiles' column split -- wave dw decodes both k-tiles of n-tiles 2 dw and 2 dw + 1 (the weights of
-    // its own 32 output columns; k-tile lane >> 5, n-tile 2 dw + ((lane >> 4) & 1)) instead of the four n-tiles above.
-    __device__ __forceinline__ Decoder(const GemmParams& p, const Tile& t, int dw, int lane, int num_kb,
-                                       bool cols = false)
+    __device__ __forceinline__ Decoder(const GemmParams& p, const Tile& t, int dw, int lane, int num_kb)
     {
         const int j16 = lane & 15;
         const int ta = j16 >> 1;
         tb = j16 & 1;
-        const int kt = cols ? (lane >> 5) : (dw >> 1);
-        const int nt8 = cols ? 2 * dw + ((lane >> 4) & 1) : 4 * (dw & 1) + (lane >> 4);
+        const int kt = dw >> 1;
+        const int nt8 = 4 * (dw & 1) + (lane >> 4);
         stage_bytes = 2 * p.tiles_n * NDW * 4;
-        const int64_t first = cols ? ((int64_t) (2 * t.kb0) * p.tiles_n + t.nt * 8 + 2 * dw) * NDW
-                                   : ((int64_t) (2 * t.kb0 + kt) * p.tiles_n + t.nt * 8 + 4 * (dw & 1)) * NDW;
+        const int64_t first = ((int64_t) (2 * t.kb0 + kt) * p.tiles_n + t.nt * 8 + 4 * (dw & 1)) * NDW;
         raw = buffer_rsrc(t.packed + first, ((int64_t) (p.size_k >> 4) * p.tiles_n * NDW - first) * 4);
         last_kb = num_kb - 1;
-        const int tile_off = cols ? (kt * p.tiles_n + ((lane >> 4) & 1)) * NDW : (lane >> 4) * NDW;
+        const int tile_off = (lane >> 4) * NDW;
         if constexpr (BITS == 3)
         {
             const int d0 = (16 * j16 * BITS + BITS - 16) >> 5;  // dword of the first window bit (may be -1)
@@ -281,43 +307,20 @@ struct Decoder
         const int so = min(kb, last_kb) * stage_bytes;
         if constexpr (BITS == 4)
         {
-            const auto v = __builtin_amdgcn_raw_buffer_load_b64(raw, off[0], so, AUX);
+            const auto v = __builtin_amdgcn_raw_buffer_load_b64(raw, off[0], so, 0);
             r[0] = v[0];
             r[1] = v[1];
         }
         else
         {
             #pragma unroll
-            for (int i = 0; i < NR; ++i) r[i] = __builtin_amdgcn_raw_buffer_load_b32(raw, off[i], so, AUX);
+            for (int i = 0; i < NR; ++i) r[i] = __builtin_amdgcn_raw_buffer_load_b32(raw, off[i], so, 0);
         }
     }
     __device__ __forceinline__ void decode(const uint32_t (&r)[NR], Out& o) const
     {
-        Chunk4& c0 = o.c[0];
-        Chunk4& c1 = o.c[1];
-        if constexpr (BITS == 4)
-        {
-            const uint32_t prev = prev_in_row(r[1]);
-            c0 = decode_chunk<4, 20>(prev, r[0]);
-            c1 = decode_chunk<4, 20>(r[0], r[1]);
-        }
-        else if constexpr (BITS == 2)
-        {
-            const uint32_t prev = prev_in_row(r[0]);
-            c0 = decode_chunk<2, 18>(prev, r[0]);
-            c1 = decode_chunk<2, 2>(r[0], r[0]);              // window ends inside r[0]
-        }
-        else
-        {
-            // chunk pair j16: windows start 19 / 43 bits (j16 even) or 3 / 27 bits (odd) into dw_off[0]. Even lanes
-            // shift their words down by 16 bits first, so both kinds decode at the compile-time offsets 3 and 27:
-            // constant shifts of a 64-bit window compile to 32-bit funnel shifts, while per-lane 64-bit shift amounts
-            // feeding the decoder's asm gave wrong results at random.
-            const uint32_t x0 = tb ? r[0] : __builtin_amdgcn_alignbit(r[1], r[0], 16);
-            const uint32_t x1 = tb ? r[1] : __builtin_amdgcn_alignbit(r[2], r[1], 16);
-            c0 = decode_chunk<3, 3>(x0, x1);
-            c1 = decode_chunk<3, 27>(x0, x1);
-        }
+        if constexpr (BITS == 3) decode_pair<3>(0u, r, tb, o);
+        else decode_pair<BITS>(prev_in_row(r[NR - 1]), r, tb, o);
     }
     __device__ __forceinline__ void store(const Out& o, uint16_t* lds) const
     {
@@ -391,6 +394,86 @@ struct Decoder1
     }
 };
 
+// Decoding straight into MFMA operands (64-row tiles): wave w decodes the weights of its own 32 output columns of each
+// stage, both k-tiles of the n-tiles 2 w and 2 w + 1, so they never pass through LDS. Lane l (i = l & 15, q = l >> 4)
+// takes column a = i & 7 and a + 8 of n-tile i >> 3 and the four rows 4 b .. and 8 + 4 b .. of k-tile q >> 1 with
+// b = q & 1: the tile's chunk pair 2 a + b, one load of the pair's own words that covers whole tiles over the wave.
+// The word before them (its 16-bit look-back) is the last word of the lane with the previous pair and comes from there
+// by ds_bpermute; a second load for it would touch every line again (a loop of nothing but these loads reads 6.7 TB/s
+// without it, 4.6 with it). Exchanging the odd 16-lane row's rows 4 .. 7 with the even row's 8 .. 11
+// (v_permlane16_swap) leaves every lane the MFMA's own k, 8 q .. + 7, so each product is summed over K exactly as
+// through the LDS tile of the other kernels. x holds column a (MFMA row i: n-tile i >> 3, column i & 7), y column a + 8.
+// NT: the raw words are loaded non-temporal (GemmParams::weights_nt).
+template <int BITS, bool NT>
+struct ColDecoder
+{
+    static constexpr int AUX = NT ? 2 : 0;                // buffer-load cache policy: 2 = non-temporal
+    static constexpr int NDW = 8 * BITS;                  // dwords per tile
+    static constexpr int NR = BITS == 2 ? 1 : 2;
+    __amdgpu_buffer_rsrc_t raw;    // based at the wave's first tile of stage 0
+    int stage_bytes, last_kb, odd;
+    uint32_t off;                  // per-lane byte offset of the own words
+    int before;                    // 4 x the lane of the previous pair
+
+    __device__ __forceinline__ ColDecoder(const GemmParams& p, const Tile& t, int wave, int lane, int num_kb)
+    {
+        const int i = lane & 15, q = lane >> 4;
+        odd = q & 1;
+        const int j = 2 * (i & 7) + odd;
+        stage_bytes = 2 * p.tiles_n * NDW * 4;
+        const int64_t first = ((int64_t) (2 * t.kb0) * p.tiles_n + t.nt * 8 + 2 * wave) * NDW;
+        raw = buffer_rsrc(t.packed + first, ((int64_t) (p.size_k >> 4) * p.tiles_n * NDW - first) * 4);
+        last_kb = num_kb - 1;
+        // 3 bits: pairs 2 a and 2 a + 1 share the dwords 3 a .. + 2, the even one owns the first two (its window starts in
+        // the dword before them), the odd one the last two (its window lies inside)
+        const int d = BITS == 3 ? 3 * (i & 7) + odd : NR * j;
+        off = 4 * (((q >> 1) * p.tiles_n + (i >> 3)) * NDW + d);
+        const int jp = (j + 15) & 15;
+        before = 4 * (16 * ((q & 2) | (jp & 1)) + (i & 8) + (jp >> 1));
+    }
+    __device__ __forceinline__ void load(int kb, uint32_t (&r)[NR]) const
+    {
+        const int so = min(kb, last_kb) * stage_bytes;
+        if constexpr (NR == 2)
+        {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b64(raw, off, so, AUX);
+            r[0] = v[0];
+            r[1] = v[1];
+        }
+        else
+            r[0] = __builtin_amdgcn_raw_buffer_load_b32(raw, off, so, AUX);
+    }
+    __device__ __forceinline__ uint32_t look_back(const uint32_t (&r)[NR]) const
+    {
+        return (uint32_t) __builtin_amdgcn_ds_bpermute(before, (int) r[NR - 1]);
+    }
+    __device__ __forceinline__ void decode(uint32_t prev, const uint32_t (&r)[NR], half8_t& x, half8_t& y) const
+    {
+        typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+        Chunks<2> o;
+        if constexpr (BITS == 3)
+        {
+            const uint32_t w[3] = {odd ? r[0] : prev, odd ? r[1] : r[0], r[1]};
+            decode_pair<3>(0u, w, odd, o);
+        }
+        else
+            decode_pair<BITS>(prev, r, odd, o);
+        auto natural = [](uint32_t& first, uint32_t& second) {
+            const auto v = __builtin_amdgcn_permlane16_swap(first, second, false, false);
+            first = v[0];
+            second = v[1];
+        };
+        Chunk4& c0 = o.c[0];
+        Chunk4& c1 = o.c[1];
+        natural(c0.w[0], c0.w[1]);
+        natural(c1.w[0], c1.w[1]);
+        natural(c0.w[2], c0.w[3]);
+        natural(c1.w[2], c1.w[3]);
+        x = __builtin_bit_cast(half8_t, u4{c0.w[0], c1.w[0], c0.w[1], c1.w[1]});
+        y = __builtin_bit_cast(half8_t, u4{c0.w[2], c1.w[2], c0.w[3], c1.w[3]});
+    }
+};
+
 // ------------------------------------------------------------------------------------------- multiplying share
 // Wave mw's (0..3) share of the MFMA work: tile rows [64 mw, 64 mw + 64) in four groups of 16 (mb).
 // v_mfma_f32_16x16x32_f16 with the decoded weights as the first operand (16 columns x 32 k) and the activations as the
@@ -440,21 +523,6 @@ struct Mma
     {
         #pragma unroll
         for (int nb = 0; nb < 8; ++nb) w[nb] = *reinterpret_cast<const half8_t*>(lds + nb * LDS_BLK + wread);
-    }
-    // The wave's own two column blocks 2 w, 2 w + 1 of the decoded stage (thin tiles' column split).
-    __device__ __forceinline__ void read_w2(const uint16_t* lds, int w, half8_t (&f)[2]) const
-    {
-        f[0] = *reinterpret_cast<const half8_t*>(lds + (2 * w) * LDS_BLK + wread);
-        f[1] = *reinterpret_cast<const half8_t*>(lds + (2 * w + 1) * LDS_BLK + wread);
-    }
-    template <int MBA>
-    __device__ __forceinline__ static void mfma2(const half8_t (&f)[2], const half8_t (&a)[4], floatx4 (&acc)[4][2])
-    {
-        #pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
-            #pragma unroll
-            for (int mb = 0; mb < MBA; ++mb)
-                acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[nb], a[mb], acc[mb][nb], 0, 0, 0);
     }
     template <int MBA, int MBN>
     __device__ __forceinline__ static void mfma(const half8_t (&w)[8], const half8_t (&a)[MBN], floatx4 (&acc)[MBN][8])
@@ -876,94 +944,126 @@ __device__ __forceinline__ void act_store(const GemmParams& p, const Tile& t, in
     }
 }
 
-// Thin tiles of at most 16 rows (one row group; the MBN == 1 kernels, which run most of the decode path's tiles): every
-// wave decodes the weights of its own 32 output columns (Decoder cols) into its part of the double-buffered stage tile
-// and multiplies the row group by them, so no wave reads weights another wave decoded and the stages need no barrier
-// (the LDS accesses of one wave complete in order). Each output element still adds its K stages in order, as the
-// shared-tile loop does, so the results are its results bit for bit. Afterwards the accumulators go through LDS so that
-// wave 0 holds the group over all 128 columns, the layout of the shared epilogue. (Taller thin tiles keep the shared
-// loop: there every wave would load all of the tile's activation rows, and a 1024-token layer ran 3.5% slower.)
-// ACT_IN: the activation operand is computed by the workgroup itself (act_load / act_store around the first
-// trellis loads) and read from LDS instead of loaded.
-// NT: the trellis words are loaded non-temporal (set where each weight is read once; GemmParams::weights_nt).
+// 64-row tiles: wave w multiplies all of the tile's row groups by its own 32 columns, whose weights it decodes straight
+// into MFMA operands (ColDecoder). The activations go through LDS in chunks of THIN_CHUNK stages: wave w loads stage w of
+// a chunk for all row groups, so each activation row is read once per workgroup, and one barrier per chunk hands it
+// over. (Every wave loading all row groups itself moves four times the bytes out of L2, which then bounds the launch: 451
+// against 348 us below. Decoding each stage once per workgroup through LDS, as the taller tiles do, makes every wave read
+// the whole 8 KB stage for one row group: at four workgroups per CU that is 96 KB per stage, 770 of ~1900 cycles.)
+// Bound: VALU issue of the decode, 70 instructions per wave and stage, at the clock the power limit leaves (1.6-1.9 GHz
+// in these launches); 8 trellis stages in flight or five workgroups per CU measured the same. 288 experts x ~28 rows, K =
+// 4096, N = 1536: 392 -> 348 us; K = 768, N = 4096 with the atomic scatter 235 -> 214 us. Afterwards the accumulators go
+// through LDS so that wave g holds row group g over all 128 columns, the layout of the shared epilogue.
+// ACT_IN (one row group): the activation operand is computed by the workgroup itself (act_load / act_store around the
+// first trellis loads) and read from LDS instead of loaded.
+template <int BITS, int MODE, int GROUPS, bool ACT_IN, bool NT>
+__device__ __forceinline__ void thin_mainloop(const GemmParams& p, const Tile& t, int wave, int lane, uint4* lds_act,
+                                              floatx4 (&acc)[4][2])
+{
+    const int num_kb = t.num_kb;
+    using Dec = ColDecoder<BITS, NT>;
+    const Dec dec(p, t, wave, lane, num_kb);
+    const Mma mm(p, t, 0, lane, num_kb, 64);
+    uint32_t raw[THIN_DEPTH][Dec::NR];
+    half8_t mine[GROUPS];                                          // the wave's stage of the chunk in flight
+    auto put = [&](int chunk) {
+        #pragma unroll
+        for (int g = 0; g < GROUPS; ++g)
+            lds_act[(((chunk & 1) * THIN_CHUNK + wave) * GROUPS + g) * 64 + lane] = __builtin_bit_cast(uint4, mine[g]);
+    };
+    ActIn ain;
+    if constexpr (ACT_IN) act_load(p, t, wave, lane, ain);
+    else mm.load_act<GROUPS>(wave, mine);
+    #pragma unroll
+    for (int s = 0; s < THIN_DEPTH; ++s) dec.load(s, raw[s]);
+    if constexpr (ACT_IN)
+    {
+        act_store(p, t, wave, lane, ain, reinterpret_cast<unsigned char*>(lds_act));
+        __syncthreads();
+    }
+    else
+    {
+        put(0);
+        mm.load_act<GROUPS>(THIN_CHUNK + wave, mine);
+    }
+    uint32_t prev = dec.look_back(raw[0]);
+    // the stages of one chunk starting at s0
+    auto trip = [&](int s0, auto n_tag) {
+        constexpr int N = decltype(n_tag)::value;
+        const int chunk = s0 / THIN_CHUNK;
+        if constexpr (!ACT_IN)
+        {
+            __syncthreads();                                       // this chunk is written, the other buffer free
+            put(chunk + 1);
+            mm.load_act<GROUPS>(s0 + 2 * THIN_CHUNK + wave, mine);
+        }
+        #pragma unroll
+        for (int u = 0; u < N; ++u)
+        {
+            const int s = s0 + u;
+            // Keep every stage's work together: the compiler otherwise decodes a whole trip's stages at its top, behind a
+            // wait for every load in flight.
+            __builtin_amdgcn_sched_barrier(0);
+            half8_t act[GROUPS];
+            #pragma unroll
+            for (int g = 0; g < GROUPS; ++g)
+                act[g] = __builtin_bit_cast(half8_t, ACT_IN ? lds_act[s * 64 + lane]
+                                                           : lds_act[(((chunk & 1) * THIN_CHUNK + u) * GROUPS + g) * 64 + lane]);
+            const uint32_t prev_next = dec.look_back(raw[(u + 1) % THIN_DEPTH]);
+            __builtin_amdgcn_sched_barrier(0);                     // the LDS reads return behind the decode
+            half8_t x, y;
+            dec.decode(prev, raw[u % THIN_DEPTH], x, y);
+            prev = prev_next;
+            dec.load(s + THIN_DEPTH, raw[u % THIN_DEPTH]);
+            #pragma unroll
+            for (int g = 0; g < GROUPS; ++g)
+            {
+                acc[g][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, act[g], acc[g][0], 0, 0, 0);
+                acc[g][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(y, act[g], acc[g][1], 0, 0, 0);
+            }
+        }
+    };
+    int s0 = 0;
+    for (; s0 + THIN_DEPTH <= num_kb; s0 += THIN_DEPTH) trip(s0, std::integral_constant<int, THIN_DEPTH>{});
+    if (s0 < num_kb) trip(s0, std::integral_constant<int, 2>{});   // num_kb is even
+}
+
 template <int BITS, int MODE, bool ACT_IN = false, bool NT = false>
 __device__ __forceinline__ void thin_tile(const GemmParams& p, const Tile& t, int group, int wave, int lane,
                                           unsigned char* lds_raw)
 {
-    uint16_t* lds_b = reinterpret_cast<uint16_t*>(lds_raw);
-    const int num_kb = t.num_kb;
-    using Dec = Decoder<BITS, NT>;
-    constexpr int NR = Dec::NR;
-    const Dec dec(p, t, wave, lane, num_kb, true);
-    const Mma mm(p, t, 0, lane, num_kb, 64);                       // the A operand of row group 0
-    // ACT_IN: stage s's activation fragment from the slice in LDS (stages past the last clamped, like the loads)
-    auto act_from_lds = [&](int s) {
-        const uint4* a = reinterpret_cast<const uint4*>(lds_raw + LDS_MAIN_BYTES);
-        return __builtin_bit_cast(half8_t, a[min(s, num_kb - 1) * 64 + lane]);
-    };
-    floatx4 acc[4][2];
-    #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) acc[0][nb] = {};
     const bool one_row = atomic_mode(MODE) && t.rows_valid == 1;   // uniform
     OneRow one{};
     if (one_row) one = one_row_inputs<MODE>(p, t, lane);           // in flight with the pipeline's first loads
-    {
-        uint32_t raw[RAW_DEPTH][NR];
-        half8_t act[ACT_DEPTH][4];
-        {
-            uint32_t r0[NR];
-            ActIn ain;
-            if constexpr (ACT_IN) act_load(p, t, wave, lane, ain);
-            dec.load(0, r0);
-            #pragma unroll
-            for (int s = 1; s <= RAW_DEPTH; ++s) dec.load(s, raw[s % RAW_DEPTH]);
-            if constexpr (ACT_IN)
-            {
-                act_store(p, t, wave, lane, ain, lds_raw + LDS_MAIN_BYTES);
-                __syncthreads();
-                #pragma unroll
-                for (int s = 0; s < ACT_DEPTH; ++s) act[s][0] = act_from_lds(s);
-            }
-            else
-                #pragma unroll
-                for (int s = 0; s < ACT_DEPTH; ++s) mm.load_act<1>(s, act[s]);
-            typename Dec::Out o;
-            dec.decode(r0, o);
-            dec.store(o, lds_b);
-        }
-        auto trip = [&](int s0, auto n_tag) {
-            constexpr int N = decltype(n_tag)::value;
-            #pragma unroll
-            for (int u = 0; u < N; ++u)
-            {
-                const int s = s0 + u;
-                half8_t f[2];
-                mm.read_w2(lds_b + (u & 1) * LDS_TILE, wave, f);  // stage s, which this wave wrote
-                typename Dec::Out o;
-                dec.decode(raw[(u + 1) % RAW_DEPTH], o);          // stage s + 1
-                Mma::mfma2<1>(f, act[u % ACT_DEPTH], acc);
-                dec.store(o, lds_b + ((u + 1) & 1) * LDS_TILE);
-                dec.load(s + 1 + RAW_DEPTH, raw[(u + 1) % RAW_DEPTH]);
-                if constexpr (ACT_IN) act[u % ACT_DEPTH][0] = act_from_lds(s + ACT_DEPTH);
-                else mm.load_act<1>(s + ACT_DEPTH, act[u % ACT_DEPTH]);
-            }
-        };
-        using full_trip = std::integral_constant<int, UNROLL>;
-        int s0 = 0;
-        if (num_kb >= UNROLL)
-        {
-            trip(0, full_trip{});
-            for (s0 = UNROLL; s0 + UNROLL <= num_kb; s0 += UNROLL) trip(s0, full_trip{});
-        }
-        if (s0 < num_kb) trip(s0, std::integral_constant<int, 2>{});
-    }
+    const int n_groups = (t.rows_valid + 15) >> 4;
+    floatx4 acc[4][2];
+    #pragma unroll
+    for (int g = 0; g < 4; ++g) acc[g][0] = acc[g][1] = floatx4{};
+    uint4* const lds_act = reinterpret_cast<uint4*>(lds_raw);
+    if constexpr (ACT_IN) thin_mainloop<BITS, MODE, 1, true, NT>(p, t, wave, lane, lds_act, acc);
+    else if (n_groups == 1) thin_mainloop<BITS, MODE, 1, false, NT>(p, t, wave, lane, lds_act, acc);
+    else if (n_groups == 2) thin_mainloop<BITS, MODE, 2, false, NT>(p, t, wave, lane, lds_act, acc);
+    else if (n_groups == 3) thin_mainloop<BITS, MODE, 3, false, NT>(p, t, wave, lane, lds_act, acc);
+    else thin_mainloop<BITS, MODE, 4, false, NT>(p, t, wave, lane, lds_act, acc);
+    __syncthreads();                                               // the activations are dead
 
-    // wave 0 collects the group: every wave puts its two column blocks in LDS
-    floatx4 full[1][8];
+    // n-tile 2 w's columns 4 kq .. + 3 are x of lane groups 0, 1 then y of 0, 1; n-tile 2 w + 1's those of 2, 3
     floatx4* xs = reinterpret_cast<floatx4*>(lds_raw);
-    __syncthreads();                                               // the stage tiles are dead
-    xs[(2 * wave) * 64 + lane] = acc[0][0];
-    xs[(2 * wave + 1) * 64 + lane] = acc[0][1];
+    #pragma unroll
+    for (int g = 0; g < 4; ++g)
+    {
+        if (g >= n_groups) break;                                  // uniform
+        #pragma unroll
+        for (int r = 0; r < 4; ++r)
+        {
+            const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[g][0][r]), __float_as_uint(acc[g][1][r]),
+                                                            false, false);
+            acc[g][0][r] = __uint_as_float(v[0]);
+            acc[g][1][r] = __uint_as_float(v[1]);
+        }
+        xs[(8 * g + 2 * wave) * 64 + lane] = acc[g][0];
+        xs[(8 * g + 2 * wave + 1) * 64 + lane] = acc[g][1];
+    }
     __syncthreads();
     if constexpr (atomic_mode(MODE))
         if (one_row)
@@ -973,21 +1073,16 @@ __device__ __forceinline__ void thin_tile(const GemmParams& p, const Tile& t, in
                 if (p.act_arrive) act_after_last_slice(p, t, group, wave, lane);   // every wave arrives
             return;
         }
-    if (wave == 0)
+    floatx4 full[1][8];
+    const bool mine = wave < n_groups;                             // uniform over the wave
+    if (mine)
         #pragma unroll
-        for (int nb = 0; nb < 8; ++nb) full[0][nb] = xs[nb * 64 + lane];
-    __syncthreads();                                               // LDS free for the epilogue's staging
+        for (int nb = 0; nb < 8; ++nb) full[0][nb] = xs[(8 * wave + nb) * 64 + lane];
+    if constexpr (atomic_mode(MODE)) __syncthreads();              // LDS free for the epilogue's staging
     float* const stage = reinterpret_cast<float*>(lds_raw) + wave * (16 * SC_ROW);
+    if (mine) epilogue<MODE, 1, 0>(p, t, wave, lane, full, stage);
     if constexpr (MODE == MODE_ATOMIC_F32)
-    {
-        if (p.act_arrive)                                          // every wave goes on to the arrival barrier
-        {
-            if (wave == 0) epilogue<MODE, 1, 0>(p, t, 0, lane, full, stage);
-            act_after_last_slice(p, t, group, wave, lane);
-            return;
-        }
-    }
-    if (wave == 0) epilogue<MODE, 1, 0>(p, t, 0, lane, full, stage);
+        if (p.act_arrive) act_after_last_slice(p, t, group, wave, lane);           // every wave arrives
 }
 
 // The main loop of a 128-, 256- or 512-row tile: the waves share each decoded stage (a barrier per stage), each
@@ -1114,7 +1209,7 @@ __device__ __forceinline__ int tile_mainloop(const GemmParams& p, const Tile& t,
 
 // 128-, 256- and 512-row tiles: the shared main loop, then every wave's epilogue over its rows.
 template <int BITS, int MODE, int MBN, int WAVES>
-__device__ __forceinline__ void shared_tile(const GemmParams& p, const Tile& t, int group, int wave, int lane,
+__device__ __forceinline__ void shared_tile(const GemmParams& p, const Tile& t, int wave, int lane,
                                             unsigned char* lds_raw, EpiLds* epi)
 {
     constexpr int GSTRIDE = WAVES == 8 ? 8 : 0;
@@ -1123,15 +1218,6 @@ __device__ __forceinline__ void shared_tile(const GemmParams& p, const Tile& t, 
 
     if constexpr (atomic_mode(MODE)) __syncthreads();            // decoded tiles are dead; LDS becomes staging
     float* const stage = reinterpret_cast<float*>(lds_raw) + wave * (16 * SC_ROW);
-    if constexpr (MODE == MODE_ATOMIC_F32 && MBN == 1 && WAVES == 4)
-    {
-        if (p.act_arrive)                                        // every wave goes on to the arrival barrier
-        {
-            if (n_w > 0) epilogue<MODE, MBN, GSTRIDE>(p, t, wave, lane, acc, stage, epi);
-            act_after_last_slice(p, t, group, wave, lane);
-            return;
-        }
-    }
     if (n_w == 0) return;
     epilogue<MODE, MBN, GSTRIDE>(p, t, wave, lane, acc, stage, epi);
 }
@@ -1142,9 +1228,8 @@ __device__ __forceinline__ void shared_tile(const GemmParams& p, const Tile& t, 
 // write stage s+1 into the other of two LDS buffers; issue loads for later stages.
 template <int WAVES> constexpr int lds_scatter_bytes() { return WAVES * 16 * SC_ROW * 4; }
 
-// MBN: 16-row groups per wave. 4 (the default): 256-row tiles, two workgroups per CU. 1 (thin): 64-row tiles of small
-// batches (those of at most 16 rows split by columns over the waves, thin_tile); a quarter of the accumulators lets four
-// workgroups share a CU.
+// MBN: 16-row groups per wave. 4 (the default): 256-row tiles, two workgroups per CU. 1 (thin): 64-row tiles
+// (thin_tile), four workgroups per CU.
 // WAVES = 8: 512-row tiles, one workgroup per CU; each wave decodes half as much of every stage (one chunk per lane),
 // so a decoded weight feeds twice the rows for the same VALU work per wave.
 template <int BITS, int MODE, bool DENSE, int MBN = 4, int WAVES = 4, bool NT = false>
@@ -1154,9 +1239,9 @@ void trellis_gemm_kernel(const GemmParams p)
 {
     static_assert(WAVES == 4 || (WAVES == 8 && MBN == 4), "8-wave workgroups run 64 rows per wave");
     constexpr int SCB = lds_scatter_bytes<WAVES>();
-    constexpr int LDS_BYTES = (atomic_mode(MODE) && SCB > LDS_MAIN_BYTES) ? SCB : LDS_MAIN_BYTES;
+    constexpr int LOOP_BYTES = MBN == 1 ? THIN_LDS_BYTES : LDS_MAIN_BYTES;
+    constexpr int LDS_BYTES = (atomic_mode(MODE) && SCB > LOOP_BYTES) ? SCB : LOOP_BYTES;
     __shared__ __align__(16) unsigned char lds_raw[LDS_BYTES];
-    __shared__ EpiLds lds_epi[WAVES];
 
     if (p.zero4 > 0)                    // every workgroup, tile or not, clears its grid-strided share up front; the
     {                                   // stores drain while the tile computes
@@ -1171,10 +1256,13 @@ void trellis_gemm_kernel(const GemmParams p)
     if (!resolve_tile<DENSE>(p, group, slot, t)) return;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (MBN == 1 && t.rows_valid <= 16)                           // uniform over the workgroup
+    if constexpr (MBN == 1)
         thin_tile<BITS, MODE, false, NT>(p, t, group, wave, lane, lds_raw);
     else
-        shared_tile<BITS, MODE, MBN, WAVES>(p, t, group, wave, lane, lds_raw, lds_epi + wave);
+    {
+        __shared__ EpiLds lds_epi[WAVES];
+        shared_tile<BITS, MODE, MBN, WAVES>(p, t, wave, lane, lds_raw, lds_epi + wave);
+    }
 }
 
 // The decode path's down GEMM with the activation pass inside (SCATTER_F32 on 64-row tiles of at most 16 rows): each
@@ -1187,8 +1275,8 @@ __global__ __launch_bounds__(256, 4)
 void trellis_gemm_actin_kernel(const GemmParams p)
 {
     constexpr int SCB = lds_scatter_bytes<4>();
-    constexpr int ACT_END = LDS_MAIN_BYTES + ACTIN_MAX_KB * 1024;
-    __shared__ __align__(16) unsigned char lds_raw[SCB > ACT_END ? SCB : ACT_END];
+    static_assert(SCB >= ACTIN_MAX_KB * 1024, "the act slice");
+    __shared__ __align__(16) unsigned char lds_raw[SCB];
     int group, slot;
     xcd_group_slot((int) blockIdx.x, p.k_split > 1 ? p.n_slots * p.k_split : p.n_slots, group, slot);
     Tile t;
