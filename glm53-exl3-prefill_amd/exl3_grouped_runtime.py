@@ -220,7 +220,10 @@ def _prefill_plan(gp, T: int, K: int, topk: int, E: int, I: int, tr: int, scatte
     """The intermediates of one grouped_prefill call of T tokens, requested in a fixed order through take(shape, dtype):
     the sorted routes, the tile tables (rows_per_tile tr, plus the thin table), and h13 / gu / act in the T16 layout."""
     R = T * topk
-    max_blocks = R // tr + E
+    # With the thin table every main-table tile holds more than THIN_ROWS rows, which bounds their number on the host: at
+    # 1024 tokens 126 entries instead of 320, and a launch over the unused ones is 12 (gate|up) or 32 (down) empty
+    # workgroups each (8.5 and 11.2 us of launches that do nothing there).
+    max_blocks = R // tr + E if not thin else min(R // tr + E, max(1, R // (THIN_ROWS + 1)))
     R16 = gp.t16_rows(R)
 
     def plan(take):

@@ -114,8 +114,8 @@ int exl3_build_tiles(const int32_t* counts, int n_experts, int tile_rows, int ma
  * Two row-tile tables for one launch pair (new): tile_rows-row tiles (128, 256 or 512), except that each expert's
  * last tile goes to a second table of thin_rows-row tiles (64) when it holds at most thin_rows rows;
  * the grouped GEMM runs the second table on its thin kernel (tile_rows 64, any mode). Tails are -1 as in
- * exl3_build_tiles; meta int32[3] = {full tiles, rows, thin tiles}. Bounds: max_full >= R/tile_rows + n_experts,
- * max_thin >= min(n_experts, R). The same launch also zeroes zero[0 .. zero_floats) (16-byte aligned, a multiple of 4
+ * exl3_build_tiles; meta int32[3] = {full tiles, rows, thin tiles}. Bounds: max_full >= min(R/tile_rows + n_experts,
+ * R/(thin_rows + 1)) (a first-table tile holds more than thin_rows rows), max_thin >= min(n_experts, R). The same launch also zeroes zero[0 .. zero_floats) (16-byte aligned, a multiple of 4
  * floats; 0 and NULL for none): the fp32 output the down GEMM's atomic scatter adds into.
  */
 int exl3_build_tiles_split(const int32_t* counts, int n_experts, int tile_rows, int thin_rows, int max_full,
