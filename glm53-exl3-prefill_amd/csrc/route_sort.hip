@@ -285,6 +285,29 @@ void sort_scatter_tiles_kernel(const void* __restrict__ ids, int ids_dtype, cons
             pre[0] += h[i].x & m; pre[1] += h[i].y & m; pre[2] += h[i].z & m; pre[3] += h[i].w & m;
         }
     }
+    if (thin_rows > 64 && wg == n_chunks)
+    {
+        // Last tiles of 65 .. thin_rows rows are faster on the thin kernel one by one, but a few of them beside many larger
+        // tiles fill the main launch's last round for nothing and lengthen the thin launch: they go to the second table
+        // when they number more than half the larger tiles (balanced routing, 288 experts, ms per layer with / without:
+        // 2048 tokens 0.777 / 0.861, 3000 0.975 / 1.211; 12 hot experts, 8192 tokens 2.06 / 2.17; Zipf routing, where
+        // they would not, 2048 tokens 0.740 / 0.706, 3000 0.930 / 0.900).
+        __shared__ int32_t s_mid, s_big;
+        if (t == 0) s_mid = s_big = 0;
+        __syncthreads();
+        int mid = 0, big = 0;
+        #pragma unroll
+        for (int j = 0; j < 4; ++j)
+        {
+            const int rem = tot[j] % tile_rows;
+            mid += rem > 64 && rem <= thin_rows;
+            big += tot[j] / tile_rows + (rem > thin_rows);
+        }
+        if (mid) atomicAdd(&s_mid, mid);
+        if (big) atomicAdd(&s_big, big);
+        __syncthreads();
+        if (2 * s_mid <= s_big) thin_rows = 64;
+    }
     int nfull[4], nthin[4];
     #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -755,14 +778,12 @@ extern "C" int exl3_build_tiles_split(const int32_t* counts, int n_experts, int 
     return hip_status("build_tiles_split");
 }
 
-extern "C" int exl3_sort_routes_split_tiles(const void* topk_ids, int ids_dtype, const void* topk_weights,
-                                            int weights_dtype, int64_t tokens, int topk, int n_experts,
-                                            int64_t* token_sorted, uint16_t* weight_sorted, int32_t* expert_of_row,
-                                            int32_t* route_index, int32_t* counts, int32_t* expert_row0,
-                                            void* workspace, size_t workspace_bytes, int tile_rows, int thin_rows,
-                                            int max_full, int max_thin, int32_t* full_expert, int32_t* full_row0,
-                                            int32_t* thin_expert, int32_t* thin_row0, int32_t* meta, float* zero,
-                                            int64_t zero_floats, void* stream)
+static int sort_and_tile(int max_thin_rows, const void* topk_ids, int ids_dtype, const void* topk_weights,
+                         int weights_dtype, int64_t tokens, int topk, int n_experts, int64_t* token_sorted,
+                         uint16_t* weight_sorted, int32_t* expert_of_row, int32_t* route_index, int32_t* counts,
+                         int32_t* expert_row0, void* workspace, size_t workspace_bytes, int tile_rows, int thin_rows,
+                         int max_full, int max_thin, int32_t* full_expert, int32_t* full_row0, int32_t* thin_expert,
+                         int32_t* thin_row0, int32_t* meta, float* zero, int64_t zero_floats, void* stream)
 {
     EXL3_CHECK(ids_dtype == EXL3_DTYPE_I64 || ids_dtype == EXL3_DTYPE_I32, "topk_ids must be int64 or int32");
     EXL3_CHECK(weights_dtype == EXL3_DTYPE_F32 || weights_dtype == EXL3_DTYPE_F16 || weights_dtype == EXL3_DTYPE_BF16,
@@ -778,8 +799,10 @@ extern "C" int exl3_sort_routes_split_tiles(const void* topk_ids, int ids_dtype,
     EXL3_CHECK(R == 0 || (topk_ids && topk_weights && token_sorted && weight_sorted && expert_of_row),
                "null pointer");
     EXL3_CHECK((reinterpret_cast<uintptr_t>(workspace) & 15) == 0, "sort workspace must be 16-byte aligned");
-    EXL3_CHECK((tile_rows == 128 || tile_rows == 256 || tile_rows == 512) && thin_rows == 64,
-               "tile_rows must be 128, 256 or 512 and thin_rows 64");
+    EXL3_CHECK((tile_rows == 128 || tile_rows == 256 || tile_rows == 512) &&
+               (thin_rows == 64 || thin_rows == max_thin_rows),
+               max_thin_rows == 64 ? "tile_rows must be 128, 256 or 512 and thin_rows 64"
+                                   : "tile_rows must be 128, 256 or 512 and thin_rows 64 or 128");
     EXL3_CHECK(max_full >= 0 && max_thin >= 0, "bad table sizes");
     EXL3_CHECK(meta && (max_full == 0 || (full_expert && full_row0)) && (max_thin == 0 || (thin_expert && thin_row0)),
                "null pointer");
@@ -799,6 +822,36 @@ extern "C" int exl3_sort_routes_split_tiles(const void* topk_ids, int ids_dtype,
         token_sorted, weight_sorted, expert_of_row, route_index, counts, expert_row0, tile_rows, thin_rows, max_full,
         max_thin, full_expert, full_row0, thin_expert, thin_row0, meta, reinterpret_cast<float4*>(zero), zero4);
     return hip_status("sort_routes_split_tiles");
+}
+
+extern "C" int exl3_sort_routes_split_tiles(const void* topk_ids, int ids_dtype, const void* topk_weights,
+                                            int weights_dtype, int64_t tokens, int topk, int n_experts,
+                                            int64_t* token_sorted, uint16_t* weight_sorted, int32_t* expert_of_row,
+                                            int32_t* route_index, int32_t* counts, int32_t* expert_row0,
+                                            void* workspace, size_t workspace_bytes, int tile_rows, int thin_rows,
+                                            int max_full, int max_thin, int32_t* full_expert, int32_t* full_row0,
+                                            int32_t* thin_expert, int32_t* thin_row0, int32_t* meta, float* zero,
+                                            int64_t zero_floats, void* stream)
+{
+    return sort_and_tile(64, topk_ids, ids_dtype, topk_weights, weights_dtype, tokens, topk, n_experts, token_sorted,
+                         weight_sorted, expert_of_row, route_index, counts, expert_row0, workspace, workspace_bytes,
+                         tile_rows, thin_rows, max_full, max_thin, full_expert, full_row0, thin_expert, thin_row0, meta,
+                         zero, zero_floats, stream);
+}
+
+extern "C" int exl3_sort_routes_tail_tiles(const void* topk_ids, int ids_dtype, const void* topk_weights,
+                                            int weights_dtype, int64_t tokens, int topk, int n_experts,
+                                            int64_t* token_sorted, uint16_t* weight_sorted, int32_t* expert_of_row,
+                                            int32_t* route_index, int32_t* counts, int32_t* expert_row0,
+                                            void* workspace, size_t workspace_bytes, int tile_rows, int thin_rows,
+                                            int max_full, int max_thin, int32_t* full_expert, int32_t* full_row0,
+                                            int32_t* thin_expert, int32_t* thin_row0, int32_t* meta, float* zero,
+                                            int64_t zero_floats, void* stream)
+{
+    return sort_and_tile(128, topk_ids, ids_dtype, topk_weights, weights_dtype, tokens, topk, n_experts, token_sorted,
+                         weight_sorted, expert_of_row, route_index, counts, expert_row0, workspace, workspace_bytes,
+                         tile_rows, thin_rows, max_full, max_thin, full_expert, full_row0, thin_expert, thin_row0, meta,
+                         zero, zero_floats, stream);
 }
 
 extern "C" int exl3_build_blocks(const int32_t* counts, int n_experts, int max_blocks,

@@ -958,22 +958,33 @@ __device__ __forceinline__ void act_store(const GemmParams& p, const Tile& t, in
 // first trellis loads) and read from LDS instead of loaded.
 template <int BITS, int MODE, int GROUPS, bool ACT_IN, bool NT>
 __device__ __forceinline__ void thin_mainloop(const GemmParams& p, const Tile& t, int wave, int lane, uint4* lds_act,
-                                              floatx4 (&acc)[4][2])
+                                              floatx4 (&acc)[GROUPS][2])
 {
     const int num_kb = t.num_kb;
     using Dec = ColDecoder<BITS, NT>;
     const Dec dec(p, t, wave, lane, num_kb);
-    const Mma mm(p, t, 0, lane, num_kb, 64);
+    // Up to four row groups: chunks of four stages, wave w loading stage w of a chunk for all groups. More: chunks of two
+    // stages, wave w loading groups w and w + 4 of every stage. SLOTS stages of SLOT_GROUPS groups in LDS: two chunks.
+    constexpr bool TALL = GROUPS > 4;
+    constexpr int CHUNK = TALL ? 2 : THIN_CHUNK, SLOTS = 2 * CHUNK;
+    constexpr int MINE = TALL ? 2 : GROUPS, SLOT_GROUPS = TALL ? 8 : GROUPS;
+    static_assert(SLOTS * SLOT_GROUPS * 1024 <= THIN_LDS_BYTES, "activation chunks");
+    const Mma mm = TALL ? Mma(p, t, wave, lane, num_kb, 64, 4) : Mma(p, t, 0, lane, num_kb, 64);
     uint32_t raw[THIN_DEPTH][Dec::NR];
-    half8_t mine[GROUPS];                                          // the wave's stage of the chunk in flight
-    auto put = [&](int chunk) {
+    half8_t mine[MINE];                                            // what the wave has in flight for a later chunk
+    auto put = [&](int s) {                                        // TALL: stage s; else the wave's stage of chunk s / CHUNK
         #pragma unroll
-        for (int g = 0; g < GROUPS; ++g)
-            lds_act[(((chunk & 1) * THIN_CHUNK + wave) * GROUPS + g) * 64 + lane] = __builtin_bit_cast(uint4, mine[g]);
+        for (int i = 0; i < MINE; ++i)
+        {
+            const int at = TALL ? (s & (SLOTS - 1)) * SLOT_GROUPS + wave + 4 * i
+                                : ((s & CHUNK) + wave) * SLOT_GROUPS + i;
+            lds_act[at * 64 + lane] = __builtin_bit_cast(uint4, mine[i]);
+        }
     };
+    auto fetch = [&](int s) { mm.load_act<MINE>(TALL ? s : s + wave, mine); };
     ActIn ain;
     if constexpr (ACT_IN) act_load(p, t, wave, lane, ain);
-    else mm.load_act<GROUPS>(wave, mine);
+    else fetch(0);
     #pragma unroll
     for (int s = 0; s < THIN_DEPTH; ++s) dec.load(s, raw[s]);
     if constexpr (ACT_IN)
@@ -984,40 +995,64 @@ __device__ __forceinline__ void thin_mainloop(const GemmParams& p, const Tile& t
     else
     {
         put(0);
-        mm.load_act<GROUPS>(THIN_CHUNK + wave, mine);
+        if constexpr (TALL)
+        {
+            fetch(1);
+            put(1);
+            fetch(2);
+        }
+        else
+            fetch(CHUNK);
     }
     uint32_t prev = dec.look_back(raw[0]);
-    // the stages of one chunk starting at s0
     auto trip = [&](int s0, auto n_tag) {
         constexpr int N = decltype(n_tag)::value;
-        const int chunk = s0 / THIN_CHUNK;
-        if constexpr (!ACT_IN)
-        {
-            __syncthreads();                                       // this chunk is written, the other buffer free
-            put(chunk + 1);
-            mm.load_act<GROUPS>(s0 + 2 * THIN_CHUNK + wave, mine);
-        }
         #pragma unroll
         for (int u = 0; u < N; ++u)
         {
             const int s = s0 + u;
+            if constexpr (!ACT_IN)
+            {
+                if (u % CHUNK == 0) __syncthreads();               // this chunk is written, the other one's slots free
+                if (TALL || u % CHUNK == 0)
+                {
+                    put(s + CHUNK);
+                    fetch(TALL ? s + CHUNK + 1 : s + 2 * CHUNK);
+                }
+            }
             // Keep every stage's work together: the compiler otherwise decodes a whole trip's stages at its top, behind a
             // wait for every load in flight.
             __builtin_amdgcn_sched_barrier(0);
             half8_t act[GROUPS];
-            #pragma unroll
-            for (int g = 0; g < GROUPS; ++g)
+            auto read = [&](int g) {
                 act[g] = __builtin_bit_cast(half8_t, ACT_IN ? lds_act[s * 64 + lane]
-                                                           : lds_act[(((chunk & 1) * THIN_CHUNK + u) * GROUPS + g) * 64 + lane]);
+                                                           : lds_act[((s & (SLOTS - 1)) * SLOT_GROUPS + g) * 64 + lane]);
+            };
+            if constexpr (!TALL)
+                #pragma unroll
+                for (int g = 0; g < GROUPS; ++g) read(g);
             const uint32_t prev_next = dec.look_back(raw[(u + 1) % THIN_DEPTH]);
             __builtin_amdgcn_sched_barrier(0);                     // the LDS reads return behind the decode
             half8_t x, y;
             dec.decode(prev, raw[u % THIN_DEPTH], x, y);
             prev = prev_next;
             dec.load(s + THIN_DEPTH, raw[u % THIN_DEPTH]);
+            if constexpr (TALL)                                    // after the decode: no registers for them before it
+            {
+                __builtin_amdgcn_sched_barrier(0);
+                #pragma unroll
+                for (int g = 0; g < 4; ++g) read(g);
+            }
             #pragma unroll
             for (int g = 0; g < GROUPS; ++g)
             {
+                if constexpr (TALL)
+                    if (g == 2)
+                    {
+                        __builtin_amdgcn_sched_barrier(0);
+                        #pragma unroll
+                        for (int h = 4; h < GROUPS; ++h) read(h);
+                    }
                 acc[g][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, act[g], acc[g][0], 0, 0, 0);
                 acc[g][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(y, act[g], acc[g][1], 0, 0, 0);
             }
@@ -1028,61 +1063,90 @@ __device__ __forceinline__ void thin_mainloop(const GemmParams& p, const Tile& t
     if (s0 < num_kb) trip(s0, std::integral_constant<int, 2>{});   // num_kb is even
 }
 
-template <int BITS, int MODE, bool ACT_IN = false, bool NT = false>
-__device__ __forceinline__ void thin_tile(const GemmParams& p, const Tile& t, int group, int wave, int lane,
-                                          unsigned char* lds_raw)
+// A thin tile of at most GROUPS row groups: the main loop, then the epilogue, four row groups (one per wave) at a time.
+template <int BITS, int MODE, int GROUPS, bool ACT_IN, bool NT>
+__device__ __forceinline__ void thin_groups(const GemmParams& p, const Tile& t, int group, int wave, int lane,
+                                            unsigned char* lds_raw)
 {
-    const bool one_row = atomic_mode(MODE) && t.rows_valid == 1;   // uniform
+    const bool one_row = GROUPS == 1 && atomic_mode(MODE) && t.rows_valid == 1;   // uniform
     OneRow one{};
     if (one_row) one = one_row_inputs<MODE>(p, t, lane);           // in flight with the pipeline's first loads
     const int n_groups = (t.rows_valid + 15) >> 4;
-    floatx4 acc[4][2];
+    floatx4 acc[GROUPS][2];
     #pragma unroll
-    for (int g = 0; g < 4; ++g) acc[g][0] = acc[g][1] = floatx4{};
-    uint4* const lds_act = reinterpret_cast<uint4*>(lds_raw);
-    if constexpr (ACT_IN) thin_mainloop<BITS, MODE, 1, true, NT>(p, t, wave, lane, lds_act, acc);
-    else if (n_groups == 1) thin_mainloop<BITS, MODE, 1, false, NT>(p, t, wave, lane, lds_act, acc);
-    else if (n_groups == 2) thin_mainloop<BITS, MODE, 2, false, NT>(p, t, wave, lane, lds_act, acc);
-    else if (n_groups == 3) thin_mainloop<BITS, MODE, 3, false, NT>(p, t, wave, lane, lds_act, acc);
-    else thin_mainloop<BITS, MODE, 4, false, NT>(p, t, wave, lane, lds_act, acc);
-    __syncthreads();                                               // the activations are dead
+    for (int g = 0; g < GROUPS; ++g) acc[g][0] = acc[g][1] = floatx4{};
+    thin_mainloop<BITS, MODE, GROUPS, ACT_IN, NT>(p, t, wave, lane, reinterpret_cast<uint4*>(lds_raw), acc);
 
-    // n-tile 2 w's columns 4 kq .. + 3 are x of lane groups 0, 1 then y of 0, 1; n-tile 2 w + 1's those of 2, 3
     floatx4* xs = reinterpret_cast<floatx4*>(lds_raw);
-    #pragma unroll
-    for (int g = 0; g < 4; ++g)
-    {
-        if (g >= n_groups) break;                                  // uniform
-        #pragma unroll
-        for (int r = 0; r < 4; ++r)
-        {
-            const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[g][0][r]), __float_as_uint(acc[g][1][r]),
-                                                            false, false);
-            acc[g][0][r] = __uint_as_float(v[0]);
-            acc[g][1][r] = __uint_as_float(v[1]);
-        }
-        xs[(8 * g + 2 * wave) * 64 + lane] = acc[g][0];
-        xs[(8 * g + 2 * wave + 1) * 64 + lane] = acc[g][1];
-    }
-    __syncthreads();
-    if constexpr (atomic_mode(MODE))
-        if (one_row)
-        {
-            if (wave == 0) one_row_epilogue<MODE>(p, t, lane, reinterpret_cast<const float*>(lds_raw), one);
-            if constexpr (MODE == MODE_ATOMIC_F32)
-                if (p.act_arrive) act_after_last_slice(p, t, group, wave, lane);   // every wave arrives
-            return;
-        }
-    floatx4 full[1][8];
-    const bool mine = wave < n_groups;                             // uniform over the wave
-    if (mine)
-        #pragma unroll
-        for (int nb = 0; nb < 8; ++nb) full[0][nb] = xs[(8 * wave + nb) * 64 + lane];
-    if constexpr (atomic_mode(MODE)) __syncthreads();              // LDS free for the epilogue's staging
     float* const stage = reinterpret_cast<float*>(lds_raw) + wave * (16 * SC_ROW);
-    if (mine) epilogue<MODE, 1, 0>(p, t, wave, lane, full, stage);
+    // row groups g0 .. g0 + 3 into LDS, in the layout of the shared epilogue: n-tile 2 w's columns 4 kq .. + 3 are x of lane
+    // groups 0, 1 then y of 0, 1; n-tile 2 w + 1's those of 2, 3
+    auto hand_over = [&](auto g0_tag) {
+        constexpr int G0 = decltype(g0_tag)::value;
+        #pragma unroll
+        for (int i = 0; i < 4 && G0 + i < GROUPS; ++i)
+        {
+            floatx4 (&a)[2] = acc[G0 + i];
+            #pragma unroll
+            for (int r = 0; r < 4; ++r)
+            {
+                const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[0][r]), __float_as_uint(a[1][r]), false,
+                                                                false);
+                a[0][r] = __uint_as_float(v[0]);
+                a[1][r] = __uint_as_float(v[1]);
+            }
+            xs[(8 * i + 2 * wave) * 64 + lane] = a[0];
+            xs[(8 * i + 2 * wave + 1) * 64 + lane] = a[1];
+        }
+    };
+    __syncthreads();                                               // the activations are dead
+    hand_over(std::integral_constant<int, 0>{});
+    static_for<(GROUPS + 3) / 4>([&](auto round_tag) {
+        constexpr int G0 = 4 * decltype(round_tag)::value;
+        constexpr bool LAST = G0 + 4 >= GROUPS;
+        if (G0 >= n_groups) return;                                // uniform
+        __syncthreads();
+        if constexpr (GROUPS == 1 && atomic_mode(MODE))
+            if (one_row)
+            {
+                if (wave == 0) one_row_epilogue<MODE>(p, t, lane, reinterpret_cast<const float*>(lds_raw), one);
+                return;
+            }
+        floatx4 full[1][8];
+        const bool mine = G0 + wave < n_groups;                    // uniform over the wave
+        if (mine)
+            #pragma unroll
+            for (int nb = 0; nb < 8; ++nb) full[0][nb] = xs[(8 * wave + nb) * 64 + lane];
+        if constexpr (atomic_mode(MODE) || !LAST) __syncthreads(); // read: LDS free for the staging or the next four groups
+        if constexpr (!atomic_mode(MODE) && !LAST) hand_over(std::integral_constant<int, G0 + 4>{});
+        if (mine) epilogue<MODE, 1, 0>(p, t, G0 + wave, lane, full, stage);
+        if constexpr (atomic_mode(MODE) && !LAST)
+        {
+            __syncthreads();
+            hand_over(std::integral_constant<int, G0 + 4>{});
+        }
+    });
     if constexpr (MODE == MODE_ATOMIC_F32)
         if (p.act_arrive) act_after_last_slice(p, t, group, wave, lane);           // every wave arrives
+}
+
+// TALL: tiles of up to 128 rows (eight row groups) instead of 64.
+template <int BITS, int MODE, bool ACT_IN, bool NT, bool TALL>
+__device__ __forceinline__ void thin_tile(const GemmParams& p, const Tile& t, int group, int wave, int lane,
+                                          unsigned char* lds_raw)
+{
+    const int n_groups = (t.rows_valid + 15) >> 4;                 // uniform
+    if constexpr (ACT_IN)
+        thin_groups<BITS, MODE, 1, true, NT>(p, t, group, wave, lane, lds_raw);
+    else if (n_groups == 1) thin_groups<BITS, MODE, 1, false, NT>(p, t, group, wave, lane, lds_raw);
+    else if (n_groups == 2) thin_groups<BITS, MODE, 2, false, NT>(p, t, group, wave, lane, lds_raw);
+    else if (n_groups == 3) thin_groups<BITS, MODE, 3, false, NT>(p, t, group, wave, lane, lds_raw);
+    else if (!TALL || n_groups == 4) thin_groups<BITS, MODE, 4, false, NT>(p, t, group, wave, lane, lds_raw);
+    else if constexpr (TALL)
+    {
+        if (n_groups <= 6) thin_groups<BITS, MODE, 6, false, NT>(p, t, group, wave, lane, lds_raw);
+        else thin_groups<BITS, MODE, 8, false, NT>(p, t, group, wave, lane, lds_raw);
+    }
 }
 
 // The main loop of a 128-, 256- or 512-row tile: the waves share each decoded stage (a barrier per stage), each
@@ -1228,8 +1292,9 @@ __device__ __forceinline__ void shared_tile(const GemmParams& p, const Tile& t, 
 // write stage s+1 into the other of two LDS buffers; issue loads for later stages.
 template <int WAVES> constexpr int lds_scatter_bytes() { return WAVES * 16 * SC_ROW * 4; }
 
-// MBN: 16-row groups per wave. 4 (the default): 256-row tiles, two workgroups per CU. 1 (thin): 64-row tiles
-// (thin_tile), four workgroups per CU.
+// MBN: 16-row groups per wave. 4 (the default): 256-row tiles, two workgroups per CU. 1 and 2: 64- and 128-row tiles
+// (thin_tile), four workgroups per CU (three, without the 8-13 registers that eight row groups spill at four, ran the
+// 128-row tables 3-4% slower).
 // WAVES = 8: 512-row tiles, one workgroup per CU; each wave decodes half as much of every stage (one chunk per lane),
 // so a decoded weight feeds twice the rows for the same VALU work per wave.
 template <int BITS, int MODE, bool DENSE, int MBN = 4, int WAVES = 4, bool NT = false>
@@ -1239,7 +1304,7 @@ void trellis_gemm_kernel(const GemmParams p)
 {
     static_assert(WAVES == 4 || (WAVES == 8 && MBN == 4), "8-wave workgroups run 64 rows per wave");
     constexpr int SCB = lds_scatter_bytes<WAVES>();
-    constexpr int LOOP_BYTES = MBN == 1 ? THIN_LDS_BYTES : LDS_MAIN_BYTES;
+    constexpr int LOOP_BYTES = MBN <= 2 ? THIN_LDS_BYTES : LDS_MAIN_BYTES;
     constexpr int LDS_BYTES = (atomic_mode(MODE) && SCB > LOOP_BYTES) ? SCB : LOOP_BYTES;
     __shared__ __align__(16) unsigned char lds_raw[LDS_BYTES];
 
@@ -1256,8 +1321,8 @@ void trellis_gemm_kernel(const GemmParams p)
     if (!resolve_tile<DENSE>(p, group, slot, t)) return;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if constexpr (MBN == 1)
-        thin_tile<BITS, MODE, false, NT>(p, t, group, wave, lane, lds_raw);
+    if constexpr (MBN <= 2)
+        thin_tile<BITS, MODE, false, NT, MBN == 2>(p, t, group, wave, lane, lds_raw);
     else
     {
         __shared__ EpiLds lds_epi[WAVES];
@@ -1283,7 +1348,7 @@ void trellis_gemm_actin_kernel(const GemmParams p)
     if (!resolve_tile<false>(p, group, slot, t)) return;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    thin_tile<BITS, MODE_SCATTER_F32, true, NT>(p, t, group, wave, lane, lds_raw);
+    thin_tile<BITS, MODE_SCATTER_F32, true, NT, false>(p, t, group, wave, lane, lds_raw);
 }
 
 template <int BITS>
@@ -1360,8 +1425,10 @@ int launch_gemm_kpair(const GemmParams& p, hipStream_t s)
     return fail("internal: K-pair launch for mode %d", MODE);
 }
 
-// 512-row tiles run the 8-wave variant, 128- and 256-row tiles the 4-wave kernel (the only one built for ATOMIC_F32,
-// whose split-K launches serve small batches), 64-row tiles the thin 4-wave variant.
+// 512-row tiles run the 8-wave variant, 256-row tiles the 4-wave kernel, 64- and 128-row tiles the thin one, which
+// decodes a tile's weights with half the instructions' waiting and no LDS traffic for them: 288 tiles of 72 / 96 / 128
+// rows, gate|up 547 / 648 / 676 us on the 4-wave kernel against 504 / 508 / 573, down 373 / 414 / 456 against 331 / 350 /
+// 407. (ATOMIC_F32 has no 8-wave kernel: its split-K launches serve small batches.)
 template <int BITS, int MODE, bool DENSE>
 int launch_gemm(const GemmParams& p, hipStream_t s)
 {
@@ -1369,15 +1436,21 @@ int launch_gemm(const GemmParams& p, hipStream_t s)
     const int64_t grid = (int64_t) groups8 * p.n_slots * (p.k_split > 1 ? p.k_split : 1);
     if (grid == 0) return EXL3_OK;
     if (grid > 0x7FFFFFFF) return fail("grid too large");
-    if (p.tile_rows == 64)
+    if (p.tile_rows <= 128)
     {
         if constexpr (!DENSE)
-            if (p.weights_nt)
-            {
+        {
+            if (p.weights_nt && p.tile_rows == 64)
                 trellis_gemm_kernel<BITS, MODE, DENSE, 1, 4, true><<<(unsigned) grid, 256, 0, s>>>(p);
-                return EXL3_OK;
-            }
-        trellis_gemm_kernel<BITS, MODE, DENSE, 1><<<(unsigned) grid, 256, 0, s>>>(p);
+            else if (p.tile_rows == 64)
+                trellis_gemm_kernel<BITS, MODE, DENSE, 1><<<(unsigned) grid, 256, 0, s>>>(p);
+            else if (p.weights_nt)
+                trellis_gemm_kernel<BITS, MODE, DENSE, 2, 4, true><<<(unsigned) grid, 256, 0, s>>>(p);
+            else
+                trellis_gemm_kernel<BITS, MODE, DENSE, 2><<<(unsigned) grid, 256, 0, s>>>(p);
+        }
+        else
+            trellis_gemm_kernel<BITS, MODE, DENSE, 1><<<(unsigned) grid, 256, 0, s>>>(p);
         return EXL3_OK;
     }
     if constexpr (MODE == MODE_ATOMIC_F32)

@@ -279,7 +279,8 @@ int grouped_gemm_split(const uint16_t* a, int64_t a_rows, int size_k, int a_layo
     // Thin tables (64-row tiles: each expert's small last tile) in the store modes, the prefill's thin launches, read
     // each tail expert's weights once: loaded non-temporal, they leave the caches to the data that is read again
     // (headline 2.083-2.096 vs 2.097-2.108 ms per layer over six alternating runs, most of it in the combine that
-    // follows). The decode path chooses per call (weights_nt).
+    // follows). exl3_grouped_gemm_once says so of a 128-row table too, except for the atomic scatter, where it measured
+    // within noise; the decode path chooses per call (weights_nt).
     p.weights_nt = (weights_nt || (tile_rows == 64 && (mode == EXL3_GEMM_STORE_F16 || mode == EXL3_GEMM_STORE_F16_T16 ||
                                                        mode == EXL3_GEMM_STORE_ROUTE_F32))) ? 1 : 0;
     if (act && act->gu_in)
@@ -381,6 +382,24 @@ extern "C" int exl3_grouped_gemm_clear(const uint16_t* a, int64_t a_rows, int si
                               tiles_n, bits, svh_gate, svh_up, svh_stride, block_expert, block_row0, max_blocks,
                               tile_rows, counts, expert_row0, n_experts, token_sorted, route_weight, route_index, out,
                               out_rows, mode, k_split, nullptr, as_stream(stream), zero, zero_floats);
+}
+
+extern "C" int exl3_grouped_gemm_once(const uint16_t* a, int64_t a_rows, int size_k, int a_layout,
+                                      const uint16_t* packed_gate, const uint16_t* packed_up,
+                                      int64_t expert_stride_words, int tiles_k, int tiles_n, int bits,
+                                      const uint16_t* svh_gate, const uint16_t* svh_up, int64_t svh_stride,
+                                      const int32_t* block_expert, const int32_t* block_row0, int max_blocks,
+                                      int tile_rows, const int32_t* counts, const int32_t* expert_row0, int n_experts,
+                                      const int64_t* token_sorted, const uint16_t* route_weight,
+                                      const int32_t* route_index, void* out, int64_t out_rows, int mode, int k_split,
+                                      float* zero, int64_t zero_floats, void* stream)
+{
+    EXL3_CHECK(tile_rows == 64 || tile_rows == 128, "weights read once: tile_rows must be 64 or 128");
+    return grouped_gemm_split(a, a_rows, size_k, a_layout, packed_gate, packed_up, expert_stride_words, tiles_k,
+                              tiles_n, bits, svh_gate, svh_up, svh_stride, block_expert, block_row0, max_blocks,
+                              tile_rows, counts, expert_row0, n_experts, token_sorted, route_weight, route_index, out,
+                              out_rows, mode, k_split, nullptr, as_stream(stream), zero, zero_floats,
+                              mode != EXL3_GEMM_SCATTER_F32);
 }
 
 extern "C" int exl3_grouped_gemm_ex(const uint16_t* a, int64_t a_rows, int size_k, int a_layout,

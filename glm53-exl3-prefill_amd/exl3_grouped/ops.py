@@ -183,6 +183,28 @@ def sort_routes_split_tiles(topk_ids: torch.Tensor, topk_weights: torch.Tensor, 
                             route_index: Optional[torch.Tensor] = None) -> torch.Tensor:
     """sort_routes followed by build_tiles_split on its counts, in two launches instead of four (new): the same
     outputs bit for bit. Returns the sort workspace (first int32: the dropped routes)."""
+    return _sort_and_tile("exl3_sort_routes_split_tiles", topk_ids, topk_weights, n_experts, token_sorted, weight_sorted,
+                          expert_of_row, counts, expert_row0, full_expert, full_row0, thin_expert, thin_row0, meta,
+                          tile_rows, thin_rows, zero, workspace, route_index)
+
+
+def sort_routes_tail_tiles(topk_ids: torch.Tensor, topk_weights: torch.Tensor, n_experts: int,
+                           token_sorted: torch.Tensor, weight_sorted: torch.Tensor, expert_of_row: torch.Tensor,
+                           counts: torch.Tensor, expert_row0: torch.Tensor, full_expert: torch.Tensor,
+                           full_row0: torch.Tensor, thin_expert: torch.Tensor, thin_row0: torch.Tensor,
+                           meta: torch.Tensor, tile_rows: int = 256, thin_rows: int = 128,
+                           zero: Optional[torch.Tensor] = None, workspace: Optional[torch.Tensor] = None,
+                           route_index: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """sort_routes_split_tiles (new) that with thin_rows 128 also puts last tiles of 65 to 128 rows into the second table
+    when they number more than half the tiles of more than 128 rows."""
+    return _sort_and_tile("exl3_sort_routes_tail_tiles", topk_ids, topk_weights, n_experts, token_sorted, weight_sorted,
+                          expert_of_row, counts, expert_row0, full_expert, full_row0, thin_expert, thin_row0, meta,
+                          tile_rows, thin_rows, zero, workspace, route_index)
+
+
+def _sort_and_tile(entry: str, topk_ids, topk_weights, n_experts, token_sorted, weight_sorted, expert_of_row, counts,
+                   expert_row0, full_expert, full_row0, thin_expert, thin_row0, meta, tile_rows, thin_rows, zero,
+                   workspace, route_index) -> torch.Tensor:
     _check(topk_ids.dim() == 2 and topk_weights.shape == topk_ids.shape, "topk_ids / topk_weights must be [T, topk]")
     _check(topk_ids.dtype in (torch.int64, torch.int32), "topk_ids must be int64 or int32")
     _check(topk_weights.dtype in (torch.float32, torch.float16, torch.bfloat16),
@@ -214,7 +236,7 @@ def sort_routes_split_tiles(topk_ids: torch.Tensor, topk_weights: torch.Tensor, 
         workspace = torch.empty(need, dtype=torch.uint8, device=dev)
     _check(workspace.numel() * workspace.element_size() >= need, "sort workspace too small")
     with _On(dev) as s:
-        _lib.call("exl3_sort_routes_split_tiles", _p(topk_ids), _DT[topk_ids.dtype], _p(topk_weights),
+        _lib.call(entry, _p(topk_ids), _DT[topk_ids.dtype], _p(topk_weights),
                   _DT[topk_weights.dtype], T, k, n_experts, _p(token_sorted), _p(weight_sorted), _p(expert_of_row),
                   _p(route_index), _p(counts), _p(expert_row0), _p(workspace),
                   workspace.numel() * workspace.element_size(), int(tile_rows), int(thin_rows), full_expert.numel(),
@@ -297,17 +319,20 @@ def grouped_gemm(a: torch.Tensor, packed_gate: torch.Tensor, packed_up: Optional
                  block_row0: torch.Tensor, counts: torch.Tensor, expert_row0: torch.Tensor,
                  token_sorted: Optional[torch.Tensor], route_weight: Optional[torch.Tensor], out: torch.Tensor,
                  mode: int, route_index: Optional[torch.Tensor] = None, tile_rows: int = 128, a_layout: int = 0,
-                 a_rows: Optional[int] = None, k_split: int = 1, zero: Optional[torch.Tensor] = None) -> None:
+                 a_rows: Optional[int] = None, k_split: int = 1, zero: Optional[torch.Tensor] = None,
+                 weights_once: bool = False) -> None:
     """kernel/exl3_grouped_prefill.cu:326-378. mode 0: fp16 store; mode 1: fp32 atomic scatter into
     out[token_sorted[r]]; mode 2 (new): fp32 store of the weighted row into out[route_index[r]] (out [T*topk, N]),
     summed per token by combine_routes in a fixed order; mode 3 (new): fp32 atomic add of the unweighted row into
     out[r] (out [rows, n_tensors*N], caller-zeroed); mode 4 (new): mode 0 into a T16-layout out (what act_had reads
     with gu_layout=1). tile_rows (new): rows per block-table entry, 128 for
     build_blocks' table (the reference's), 256 or 512 for a build_tiles(..., 256 | 512) table (512 runs the 8-wave
-    kernel), 64 (a thin kernel for small tiles, 16 rows per wave). a_layout (new): 0 row-major a,
+    kernel), 64 for small tiles (64- and 128-row tiles run the thin kernel). a_layout (new): 0 row-major a,
     1 T16 (a from row_had / act_had with dst_layout=1; a_rows gives its logical rows). k_split (new): slices of K
     whose partial products are added into out (modes 1 and 3 only). zero (new, optional fp32 contiguous, numel % 4 ==
-    0, not overlapping a or out): cleared by the same launch, e.g. the output a later mode-1 launch adds into."""
+    0, not overlapping a or out): cleared by the same launch, e.g. the output a later mode-1 launch adds into.
+    weights_once (new; tile_rows 64 or 128): the table holds at most one tile per expert, so the weights may be loaded
+    non-temporal."""
     _check(int(tile_rows) in (64, 128, 256, 512), "tile_rows must be 64, 128, 256 or 512")
     _check(int(k_split) >= 1 and int(k_split) <= a.size(1) // 64, "k_split must be in [1, K / 64]")
     _check(int(k_split) == 1 or mode in (1, 3), "k_split > 1 needs mode 1 or 3")
@@ -373,7 +398,9 @@ def grouped_gemm(a: torch.Tensor, packed_gate: torch.Tensor, packed_up: Optional
             _p(route_weight) if weighted else None, _p(route_index) if mode == 2 else None, _p(out), out.size(0), mode,
             int(k_split))
     with _On(dev) as s:
-        if zero is None:
+        if weights_once:
+            _lib.call("exl3_grouped_gemm_once", *args, _p(zero), 0 if zero is None else zero.numel(), s)
+        elif zero is None:
             _lib.call("exl3_grouped_gemm_split", *args, s)
         else:
             _lib.call("exl3_grouped_gemm_clear", *args, _p(zero), zero.numel(), s)

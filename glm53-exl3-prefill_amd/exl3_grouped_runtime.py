@@ -11,8 +11,8 @@ Expert-parallel calls (layer.expert_map set) and layers without w13_trellis keep
 Env:
   EXL3_GROUPED_PREFILL=1     enable (read by the hook)
   EXL3_GROUPED_DECODE=0      leave decode calls (tokens <= cap) to the original path (default: moe_decode)
-  EXL3_GROUPED_THIN=0        run every expert tile on the main GEMM kernel (default: an expert's last tile of <= 64
-                             rows runs on the thin kernel, four workgroups per CU, in a second launch)
+  EXL3_GROUPED_THIN=0        run every expert tile on the main GEMM kernel (default: an expert's small last tile runs on
+                             the thin kernel, four workgroups per CU, in a second launch)
   EXL3_GROUPED_SCATTER=...   down-projection output: "atomic" (fp32 atomic scatter by token, the reference's
                              method), "combine" (per-route fp32 rows + a fixed-order sum per token: deterministic) or
                              "auto" (the default: combine for chunks of >= COMBINE_MIN_ROUTES routes, else atomic)
@@ -101,7 +101,9 @@ def thin_tiles_enabled() -> bool:
     return os.environ.get("EXL3_GROUPED_THIN", "1") != "0"
 
 
-THIN_ROWS = 64
+# Rows of the tail table: each expert's last tile of at most 64, or where they are many at most THIN_ROWS, rows runs on
+# the thin kernel (sort_routes_tail_tiles).
+THIN_ROWS = 128
 
 # The prefill intermediates (sorted routes, tile tables, h13, gu, act: ~0.85 GB at 8192 tokens; with the combine output
 # also the per-route fp32 rows, 1.07 GB more at H = 4096) live in one buffer per device, reused by every call: steady-state
@@ -220,10 +222,10 @@ def _prefill_plan(gp, T: int, K: int, topk: int, E: int, I: int, tr: int, scatte
     """The intermediates of one grouped_prefill call of T tokens, requested in a fixed order through take(shape, dtype):
     the sorted routes, the tile tables (rows_per_tile tr, plus the thin table), and h13 / gu / act in the T16 layout."""
     R = T * topk
-    # With the thin table every main-table tile holds more than THIN_ROWS rows, which bounds their number on the host: at
-    # 1024 tokens 126 entries instead of 320, and a launch over the unused ones is 12 (gate|up) or 32 (down) empty
+    # With the tail table every main-table tile holds more than 64 rows (or is full), which bounds their number on the host:
+    # at 1024 tokens 126 entries instead of 320, and a launch over the unused ones is 12 (gate|up) or 32 (down) empty
     # workgroups each (8.5 and 11.2 us of launches that do nothing there).
-    max_blocks = R // tr + E if not thin else min(R // tr + E, max(1, R // (THIN_ROWS + 1)))
+    max_blocks = R // tr + E if not thin else min(R // tr + E, max(1, R // 65))
     R16 = gp.t16_rows(R)
 
     def plan(take):
@@ -252,7 +254,7 @@ def grouped_prefill(x2d: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
     stage_events: if a list is given, a timing event recorded on the current stream after each stage is appended
     as (stage name, event), after a leading ("start", event).
     scatter: "atomic", "combine" or "auto" (default: EXL3_GROUPED_SCATTER, else "auto"; resolve_scatter).
-    thin_tiles: run each expert's last tile of <= 64 rows on the thin GEMM kernel (default: EXL3_GROUPED_THIN, else
+    thin_tiles: run each expert's small last tile on the thin GEMM kernel (default: EXL3_GROUPED_THIN, else
     on). Same arithmetic per row, so the same result.
     out_dtype (new): return out in this dtype (bf16 or fp16), as out.to(out_dtype) of the fp32 result would; the combine
     method writes it directly (no fp32 round trip through memory), the atomic scatter casts its fp32 target."""
@@ -287,14 +289,14 @@ def grouped_prefill(x2d: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
     block_expert, block_row0, meta = B["block_expert"], B["block_row0"], B["meta"]
     out = None
     if thin:
-        # the sort and the two tile tables (each expert's last tile of <= 64 rows goes to a second table, run by the
-        # thin kernel) in two launches; the fp32 output the atomic down scatter adds into is cleared by the gate|up
+        # the sort and the two tile tables (each expert's small last tile goes to a second table, run by
+        # the thin kernel) in two launches; the fp32 output the atomic down scatter adds into is cleared by the gate|up
         # launch, whose MFMA-bound workgroups hide the stores
         thin_expert, thin_row0 = B["thin_expert"], B["thin_row0"]
         out = torch.empty(T, K, dtype=torch.float32, device=dev) if scatter == "atomic" else None
-        gp.sort_routes_split_tiles(ids, weights, E, token_sorted, weight_sorted, expert_of_row, counts, expert_row0,
-                                   block_expert, block_row0, thin_expert, thin_row0, meta, tr, THIN_ROWS,
-                                   workspace=B["sort_ws"], route_index=route_index)
+        gp.sort_routes_tail_tiles(ids, weights, E, token_sorted, weight_sorted, expert_of_row, counts, expert_row0,
+                                  block_expert, block_row0, thin_expert, thin_row0, meta, tr, THIN_ROWS,
+                                  workspace=B["sort_ws"], route_index=route_index)
         mark("sort_routes")                               # sort and tile tables
     else:
         gp.sort_routes(ids, weights, E, token_sorted, weight_sorted, expert_of_row, counts, expert_row0,
@@ -311,7 +313,7 @@ def grouped_prefill(x2d: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
                     tile_rows=tr, a_layout=1, a_rows=R, zero=out if thin else None)
     if thin:
         gp.grouped_gemm(h13, *w13, thin_expert, thin_row0, counts, expert_row0, token_sorted, weight_sorted, gu, 4,
-                        tile_rows=THIN_ROWS, a_layout=1, a_rows=R)
+                        tile_rows=THIN_ROWS, a_layout=1, a_rows=R, weights_once=True)
     mark("gemm_gate_up")
     act = B["act"]
     gp.act_had(gu, act, expert_of_row, layer.w2_suh, float(limit), dst_layout=1, gu_layout=1, rows=R)
@@ -326,7 +328,7 @@ def grouped_prefill(x2d: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
         if thin:
             gp.grouped_gemm(act, layer.w2_trellis, None, layer.w2_svh, None,
                             thin_expert, thin_row0, counts, expert_row0, token_sorted, weight_sorted, out, 1,
-                            tile_rows=THIN_ROWS, a_layout=1, a_rows=R)
+                            tile_rows=THIN_ROWS, a_layout=1, a_rows=R, weights_once=True)
         mark("gemm_down_scatter")
         return out if out_dtype is None else out.to(out_dtype)
     partial = B["partial"]
@@ -336,7 +338,7 @@ def grouped_prefill(x2d: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
     if thin:
         gp.grouped_gemm(act, layer.w2_trellis, None, layer.w2_svh, None,
                         thin_expert, thin_row0, counts, expert_row0, None, weight_sorted, partial, 2,
-                        route_index=route_index, tile_rows=THIN_ROWS, a_layout=1, a_rows=R)
+                        route_index=route_index, tile_rows=THIN_ROWS, a_layout=1, a_rows=R, weights_once=True)
     mark("gemm_down_routes")
     direct = out_dtype in (torch.bfloat16, torch.float16)
     out = torch.empty(T, K, dtype=out_dtype if direct else torch.float32, device=dev)

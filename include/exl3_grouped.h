@@ -115,8 +115,9 @@ int exl3_build_tiles(const int32_t* counts, int n_experts, int tile_rows, int ma
  * last tile goes to a second table of thin_rows-row tiles (64) when it holds at most thin_rows rows;
  * the grouped GEMM runs the second table on its thin kernel (tile_rows 64, any mode). Tails are -1 as in
  * exl3_build_tiles; meta int32[3] = {full tiles, rows, thin tiles}. Bounds: max_full >= min(R/tile_rows + n_experts,
- * R/(thin_rows + 1)) (a first-table tile holds more than thin_rows rows), max_thin >= min(n_experts, R). The same launch also zeroes zero[0 .. zero_floats) (16-byte aligned, a multiple of 4
- * floats; 0 and NULL for none): the fp32 output the down GEMM's atomic scatter adds into.
+ * R/min(tile_rows, thin_rows + 1)) (a first-table tile is full or holds more than thin_rows rows), max_thin >=
+ * min(n_experts, R). The same launch also zeroes zero[0 .. zero_floats) (16-byte aligned, a multiple of 4 floats; 0 and
+ * NULL for none): the fp32 output the down GEMM's atomic scatter adds into.
  */
 int exl3_build_tiles_split(const int32_t* counts, int n_experts, int tile_rows, int thin_rows, int max_full,
                            int max_thin, int32_t* full_expert, int32_t* full_row0, int32_t* thin_expert,
@@ -135,6 +136,19 @@ int exl3_sort_routes_split_tiles(const void* topk_ids, int ids_dtype, const void
                                  int tile_rows, int thin_rows, int max_full, int max_thin, int32_t* full_expert,
                                  int32_t* full_row0, int32_t* thin_expert, int32_t* thin_row0, int32_t* meta,
                                  float* zero, int64_t zero_floats, void* stream);
+
+/*
+ * exl3_sort_routes_split_tiles that also takes thin_rows 128 (new; a table for grouped GEMMs with tile_rows 128): last
+ * tiles of 65 to 128 rows go to the second table too when they number more than half the tiles of more than 128 rows,
+ * otherwise it is the table of thin_rows 64. Bound: max_full >= min(R/tile_rows + n_experts, R/min(tile_rows, 65)).
+ */
+int exl3_sort_routes_tail_tiles(const void* topk_ids, int ids_dtype, const void* topk_weights, int weights_dtype,
+                                int64_t tokens, int topk, int n_experts, int64_t* token_sorted,
+                                uint16_t* weight_sorted, int32_t* expert_of_row, int32_t* route_index,
+                                int32_t* counts, int32_t* expert_row0, void* workspace, size_t workspace_bytes,
+                                int tile_rows, int thin_rows, int max_full, int max_thin, int32_t* full_expert,
+                                int32_t* full_row0, int32_t* thin_expert, int32_t* thin_row0, int32_t* meta,
+                                float* zero, int64_t zero_floats, void* stream);
 
 /*
  * Input Hadamard (pybind op row_had, kernel/exl3_grouped_prefill.cu:101-115 and :296-311):
@@ -206,8 +220,8 @@ int exl3_grouped_gemm(const uint16_t* a, int64_t a_rows, int size_k,
  * exl3_grouped_gemm with two extensions (new): a_layout (EXL3_LAYOUT_ROWS, or EXL3_LAYOUT_T16 for an `a` written by
  * the _ex Hadamard passes) and tile_rows, the rows per block-table entry (128: the reference's build_blocks table,
  * what exl3_grouped_gemm passes; 256 or 512: a table from exl3_build_tiles(..., 256 | 512, ...); 512-row tiles run
- * an 8-wave kernel; 64: a table from exl3_build_tiles(..., 64, ...) or the thin table of exl3_build_tiles_split, run
- * by a thin kernel with 16 rows per wave). Same modes and outputs.
+ * an 8-wave kernel; 64: a table from exl3_build_tiles(..., 64, ...) or the thin table of exl3_build_tiles_split; 64- and
+ * 128-row tiles run the thin kernel). Same modes and outputs.
  */
 int exl3_grouped_gemm_ex(const uint16_t* a, int64_t a_rows, int size_k, int a_layout,
                          const uint16_t* packed_gate, const uint16_t* packed_up, int64_t expert_stride_words,
@@ -224,8 +238,7 @@ int exl3_grouped_gemm_ex(const uint16_t* a, int64_t a_rows, int size_k, int a_la
  * partial product and adds it to the output, so k_split > 1 needs an accumulating mode: EXL3_GEMM_SCATTER_F32, or
  * EXL3_GEMM_ATOMIC_F32 -- out fp32 [a_rows, n_tensors*N_each], caller-zeroed,
  *        out[r, which*N_each + n] += H128_n(a[r] @ W'_e,which) / sqrt(128) * svh_e,which[n]
- * (valid with k_split == 1 too; tile_rows 64, 128 or 256; 64 runs the thin kernel, 16 rows per wave and four
- * workgroups per CU, for small tiles).
+ * (valid with k_split == 1 too; tile_rows 64, 128 or 256).
  * 1 <= k_split <= size_k / 64; the slice count used is
  * ceil(K_stages / per_slice) with per_slice = ceil(K_stages / k_split) rounded up to even (K_stages = size_k / 32).
  */
@@ -251,6 +264,19 @@ int exl3_grouped_gemm_clear(const uint16_t* a, int64_t a_rows, int size_k, int a
                             const int64_t* token_sorted, const uint16_t* route_weight, const int32_t* route_index,
                             void* out, int64_t out_rows, int mode, int k_split, float* zero, int64_t zero_floats,
                             void* stream);
+
+/*
+ * exl3_grouped_gemm_clear for a table of at most one tile per expert (tile_rows 64 or 128; new): every expert's weights
+ * are read once, so the launch loads them non-temporal where that pays. Same outputs.
+ */
+int exl3_grouped_gemm_once(const uint16_t* a, int64_t a_rows, int size_k, int a_layout,
+                           const uint16_t* packed_gate, const uint16_t* packed_up, int64_t expert_stride_words,
+                           int tiles_k, int tiles_n, int bits, const uint16_t* svh_gate, const uint16_t* svh_up,
+                           int64_t svh_stride, const int32_t* block_expert, const int32_t* block_row0, int max_blocks,
+                           int tile_rows, const int32_t* counts, const int32_t* expert_row0, int n_experts,
+                           const int64_t* token_sorted, const uint16_t* route_weight, const int32_t* route_index,
+                           void* out, int64_t out_rows, int mode, int k_split, float* zero, int64_t zero_floats,
+                           void* stream);
 
 /*
  * Deterministic route combine (new; pairs with grouped_gemm mode 2): out[t, :] = sum_{j < topk} partial[t*topk + j, :]

@@ -1,4 +1,4 @@
-"""64-row tiles (weights decoded straight into MFMA operands, activations through LDS in four-stage chunks) against the
+"""64- and 128-row tiles (weights decoded straight into MFMA operands, activations through LDS in four-stage chunks) against the
 256-row kernel (weights decoded through LDS) bit for bit, and against the CPU oracle: row counts around every 16-row
 group, K of whole and partial chunks, every trellis width."""
 import numpy as np
@@ -29,3 +29,66 @@ def test_thin_tiles_match_256_row_tiles(dev, bits, K):
         # fp16 products are exact in fp32: what is left is the rounding of K + 128 fp32 sums per output, 2^-24 each and
         # random in sign, so sqrt(K + 128) 2^-24 <= 1.8e-6 in the 2-norm
         assert O.rel_l2(got[0], ref[:m]) < 2e-6, m
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("K", [64, 192, 768])
+def test_grouped_128_row_tiles_match_256_row_tiles(dev, bits, K):
+    """One tile per expert, row counts around every 16-row group up to 128: fp16 T16 rows of two tensors, per-route fp32
+    rows and the atomic scatter (one add per token) on a 128-row table against a 256-row one."""
+    rows = [128, 1, 16, 17, 64, 65, 80, 81, 96, 97, 112, 113, 127]
+    E, N, R = len(rows), 256, sum(rows)
+    rng = np.random.default_rng(bits * 100 + K)
+    words = torch.from_numpy(rng.integers(-32768, 32768, (E, 2, K // 16, N // 16, 16 * bits), dtype=np.int16)).to(dev)
+    svh = torch.from_numpy((rng.uniform(0.5, 1.5, (E, 2, N))).astype(np.float16)).to(dev)
+    a = torch.from_numpy(rng.standard_normal((gp.t16_rows(R), K)).astype(np.float16)).to(dev)
+    counts = torch.tensor(rows, dtype=torch.int32, device=dev)
+    row0 = (torch.cumsum(counts, 0) - counts).to(torch.int32)
+    experts = torch.arange(E, dtype=torch.int32, device=dev)
+    rw = torch.from_numpy(rng.uniform(0.1, 1, R).astype(np.float16)).to(dev)
+    route = torch.from_numpy(rng.permutation(R).astype(np.int32)).to(dev)
+    got = {}
+    for tr in (128, 256):
+        kw = dict(tile_rows=tr, a_layout=1, a_rows=R, weights_once=tr == 128)
+        gu = torch.full((gp.t16_rows(R), 2 * N), float("nan"), dtype=torch.float16, device=dev)
+        gp.grouped_gemm(a, words[:, 0], words[:, 1], svh[:, 0], svh[:, 1], experts, row0, counts, row0, None, None, gu, 4,
+                        **kw)
+        per_route = torch.full((R, N), float("nan"), dtype=torch.float32, device=dev)
+        gp.grouped_gemm(a, words[:, 0], None, svh[:, 0], None, experts, row0, counts, row0, None, rw, per_route, 2,
+                        route_index=route, **kw)
+        out = torch.zeros(R, N, dtype=torch.float32, device=dev)
+        gp.grouped_gemm(a, words[:, 0], None, svh[:, 0], None, experts, row0, counts, row0, route.long(), rw, out, 1, **kw)
+        got[tr] = [t.cpu().numpy() for t in (gu.view(torch.int16), per_route.view(torch.int32), out.view(torch.int32))]
+        assert torch.equal(out, per_route)                     # one add onto zero per row
+    for x, y in zip(got[128], got[256]):
+        assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("tile_rows,thin_rows,T", [(128, 128, 700), (256, 128, 700), (256, 128, 120), (256, 128, 4000),
+                                                   (512, 128, 700), (256, 64, 700)])
+def test_tail_tables(dev, tile_rows, thin_rows, T):
+    """sort_routes_tail_tiles' two tables against a closed form, at the smallest table the bound allows."""
+    rng = np.random.default_rng(tile_rows + thin_rows)
+    E, k = 24, 4
+    p = rng.uniform(0, 1, E) ** (1 if T > 1000 else 3)
+    ids = np.stack([rng.choice(E, k, replace=False, p=p / p.sum()) for _ in range(T)])
+    R, counts = T * k, np.bincount(ids.ravel(), minlength=E)
+    rem = counts % tile_rows
+    mid, big = ((rem > 64) & (rem <= 128)).sum(), (counts // tile_rows + (rem > 128)).sum()
+    limit = thin_rows if 2 * mid > big else 64
+    full, thin, row = [], [], 0
+    for e, c in enumerate(counts):
+        for r in range(0, c, tile_rows):
+            (thin if c - r <= limit and c - r < tile_rows else full).append((e, row + r))
+        row += c
+    mf, mt = min(R // tile_rows + E, max(1, R // min(tile_rows, 65))), min(E, R)
+    assert len(full) <= mf
+    i32 = lambda n: torch.full((n,), -7, dtype=torch.int32, device=dev)  # noqa: E731
+    fe, fr, te, tr, meta, cnt, row0, eor = i32(mf), i32(mf), i32(mt), i32(mt), i32(3), i32(E), i32(E), i32(R)
+    ts, ws = torch.empty(R, dtype=torch.int64, device=dev), torch.empty(R, dtype=torch.float16, device=dev)
+    gp.sort_routes_tail_tiles(torch.from_numpy(ids).to(dev), torch.ones(T, k, device=dev), E, ts, ws, eor, cnt, row0, fe, fr,
+                              te, tr, meta, tile_rows, thin_rows)
+    assert meta.tolist() == [len(full), R, len(thin)] and cnt.tolist() == counts.tolist()
+    for tab, e, r in ((full, fe, fr), (thin, te, tr)):
+        assert list(zip(e.tolist(), r.tolist()))[:len(tab)] == tab
+        assert (e[len(tab):] == -1).all()
