@@ -21,6 +21,17 @@ __device__ __forceinline__ uint4 pack8(const float (&x)[8])
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+// Eight packed bf16 values as fp16, each rounded to nearest even once (a bf16 tensor's cast to fp16).
+__device__ __forceinline__ uint4 f16_from_bf16(const uint4 v)
+{
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    uint32_t o[4];
+    #pragma unroll
+    for (int i = 0; i < 4; ++i)
+        o[i] = (uint32_t) f2h(__uint_as_float(w[i] << 16)) | ((uint32_t) f2h(__uint_as_float(w[i] & 0xFFFF0000u)) << 16);
+    return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
 // Butterfly stages len, 2 len, ... < end over the lane's 32 registers.
 template <int LEN0, int END>
 __device__ __forceinline__ void fwht_regs(float (&x)[32])

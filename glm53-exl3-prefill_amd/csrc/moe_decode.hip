@@ -194,8 +194,8 @@ constexpr int PREP_THREADS = 256;
 // route's row; a wave takes 16 routes x one 128-column block per step. The remaining workgroups clear two fp32
 // buffers (float4 counts na, nb).
 __global__ __launch_bounds__(PREP_THREADS)
-void decode_prep_tiny_kernel(const uint16_t* __restrict__ x, int hidden, const void* __restrict__ ids, int ids_dtype,
-                             const void* __restrict__ weights, int w_dtype, int R, int topk, int n_experts,
+void decode_prep_tiny_kernel(const uint16_t* __restrict__ x, int x_bf16, int hidden, const void* __restrict__ ids,
+                             int ids_dtype, const void* __restrict__ weights, int w_dtype, int R, int topk, int n_experts,
                              const uint16_t* __restrict__ suh, int64_t suh_stride, int max_tiles, int n_had,
                              int64_t* __restrict__ token_sorted, uint16_t* __restrict__ weight_sorted,
                              int32_t* __restrict__ expert_of_row, int32_t* __restrict__ counts,
@@ -327,7 +327,8 @@ void decode_prep_tiny_kernel(const uint16_t* __restrict__ x, int hidden, const v
         for (int k = 0; k < 4; ++k)
         {
             const int c = blk * 128 + 8 * (4 * k + cq);
-            mul8_stage1(*reinterpret_cast<const uint4*>(x + tok * hidden + c),
+            const uint4 xv = *reinterpret_cast<const uint4*>(x + tok * hidden + c);
+            mul8_stage1(x_bf16 ? f16_from_bf16(xv) : xv,
                         *reinterpret_cast<const uint4*>(suh + (int64_t) e * suh_stride + c), v + 8 * k);
         }
         had128_t16_from2_unscaled(v);
@@ -352,15 +353,17 @@ extern "C" int64_t exl3_moe_decode_workspace_bytes(int64_t tokens, int topk, int
     return decode_layout(tokens, topk, n_experts, hidden, inter).total;
 }
 
-extern "C" int exl3_moe_decode(const uint16_t* x, int64_t tokens, int hidden, const void* topk_ids, int ids_dtype,
-                               const void* topk_weights, int weights_dtype, int topk, int n_experts, int inter,
-                               int bits, const uint16_t* packed_gate, const uint16_t* packed_up,
-                               int64_t w13_expert_stride_words, const uint16_t* suh_gate, int64_t suh13_stride,
-                               const uint16_t* svh_gate, const uint16_t* svh_up, int64_t svh13_stride,
-                               const uint16_t* packed_down, int64_t w2_expert_stride_words, const uint16_t* suh_down,
-                               int64_t suh2_stride, const uint16_t* svh_down, int64_t svh2_stride, float limit,
-                               float* out, void* workspace, int64_t workspace_bytes, void* stream)
+static int moe_decode_from(int x_dtype, const uint16_t* x, int64_t tokens, int hidden, const void* topk_ids,
+                           int ids_dtype,
+                           const void* topk_weights, int weights_dtype, int topk, int n_experts, int inter,
+                           int bits, const uint16_t* packed_gate, const uint16_t* packed_up,
+                           int64_t w13_expert_stride_words, const uint16_t* suh_gate, int64_t suh13_stride,
+                           const uint16_t* svh_gate, const uint16_t* svh_up, int64_t svh13_stride,
+                           const uint16_t* packed_down, int64_t w2_expert_stride_words, const uint16_t* suh_down,
+                           int64_t suh2_stride, const uint16_t* svh_down, int64_t svh2_stride, float limit,
+                           float* out, void* workspace, int64_t workspace_bytes, void* stream)
 {
+    EXL3_CHECK(x_dtype == EXL3_DTYPE_F16 || x_dtype == EXL3_DTYPE_BF16, "x must be fp16 or bf16");
     EXL3_CHECK(tokens >= 0 && topk > 0, "bad routing shape");
     EXL3_CHECK(hidden > 0 && hidden % 128 == 0 && inter > 0 && inter % 128 == 0,
                "hidden and intermediate sizes must be multiples of 128");
@@ -405,7 +408,8 @@ extern "C" int exl3_moe_decode(const uint16_t* x, int64_t tokens, int hidden, co
         const int64_t n4 = n_out / 4 + n_gu / 4;
         const int64_t zwgs = std::min<int64_t>((n4 + PREP_THREADS - 1) / PREP_THREADS, 1024);
         decode_prep_tiny_kernel<<<(unsigned) (1 + n_had + zwgs), PREP_THREADS, 0, s>>>(
-            x, hidden, topk_ids, ids_dtype, topk_weights, weights_dtype, (int) R, topk, n_experts, suh_gate,
+            x, x_dtype == EXL3_DTYPE_BF16, hidden, topk_ids, ids_dtype, topk_weights, weights_dtype, (int) R, topk,
+            n_experts, suh_gate,
             suh13_stride, L.max_blocks, n_had, token_sorted, weight_sorted, expert_of_row, counts, expert_row0,
             block_expert, block_row0, meta, h13, reinterpret_cast<float4*>(out), n_out / 4,
             reinterpret_cast<float4*>(gu), n_gu / 4);
@@ -437,8 +441,11 @@ extern "C" int exl3_moe_decode(const uint16_t* x, int64_t tokens, int hidden, co
     }
     if (R > TINY_ROUTES)
     {
-        rc = exl3_row_had_ex(x, h13, token_sorted, expert_of_row, suh_gate, suh13_stride, hidden, R, hidden, 1,
-                             EXL3_LAYOUT_T16, stream);
+        rc = x_dtype == EXL3_DTYPE_BF16
+                 ? exl3_row_had_gather_bf16(x, h13, token_sorted, expert_of_row, suh_gate, suh13_stride, hidden, R,
+                                            hidden, stream)
+                 : exl3_row_had_ex(x, h13, token_sorted, expert_of_row, suh_gate, suh13_stride, hidden, R, hidden, 1,
+                                   EXL3_LAYOUT_T16, stream);
         if (rc) return rc;
     }
     const int target = target_workgroups();
@@ -472,6 +479,39 @@ extern "C" int exl3_moe_decode(const uint16_t* x, int64_t tokens, int hidden, co
                                    block_row0, L.max_blocks, DECODE_TILE_ROWS, counts, expert_row0, n_experts,
                                    token_sorted, weight_sorted, nullptr, out, tokens, EXL3_GEMM_SCATTER_F32,
                                    down_split, stream);
+}
+
+extern "C" int exl3_moe_decode(const uint16_t* x, int64_t tokens, int hidden, const void* topk_ids, int ids_dtype,
+                               const void* topk_weights, int weights_dtype, int topk, int n_experts, int inter,
+                               int bits, const uint16_t* packed_gate, const uint16_t* packed_up,
+                               int64_t w13_expert_stride_words, const uint16_t* suh_gate, int64_t suh13_stride,
+                               const uint16_t* svh_gate, const uint16_t* svh_up, int64_t svh13_stride,
+                               const uint16_t* packed_down, int64_t w2_expert_stride_words, const uint16_t* suh_down,
+                               int64_t suh2_stride, const uint16_t* svh_down, int64_t svh2_stride, float limit,
+                               float* out, void* workspace, int64_t workspace_bytes, void* stream)
+{
+    return moe_decode_from(EXL3_DTYPE_F16, x, tokens, hidden, topk_ids, ids_dtype, topk_weights, weights_dtype,
+                           topk, n_experts, inter, bits, packed_gate, packed_up, w13_expert_stride_words, suh_gate,
+                           suh13_stride, svh_gate, svh_up, svh13_stride, packed_down, w2_expert_stride_words,
+                           suh_down, suh2_stride, svh_down, svh2_stride, limit, out, workspace, workspace_bytes,
+                           stream);
+}
+
+extern "C" int exl3_moe_decode_dt(const void* x, int x_dtype, int64_t tokens, int hidden, const void* topk_ids,
+                                  int ids_dtype,
+                                  const void* topk_weights, int weights_dtype, int topk, int n_experts, int inter,
+                                  int bits, const uint16_t* packed_gate, const uint16_t* packed_up,
+                                  int64_t w13_expert_stride_words, const uint16_t* suh_gate, int64_t suh13_stride,
+                                  const uint16_t* svh_gate, const uint16_t* svh_up, int64_t svh13_stride,
+                                  const uint16_t* packed_down, int64_t w2_expert_stride_words, const uint16_t* suh_down,
+                                  int64_t suh2_stride, const uint16_t* svh_down, int64_t svh2_stride, float limit,
+                                  float* out, void* workspace, int64_t workspace_bytes, void* stream)
+{
+    return moe_decode_from(x_dtype, reinterpret_cast<const uint16_t*>(x), tokens, hidden, topk_ids, ids_dtype,
+                           topk_weights, weights_dtype, topk, n_experts, inter, bits, packed_gate, packed_up,
+                           w13_expert_stride_words, suh_gate, suh13_stride, svh_gate, svh_up, svh13_stride,
+                           packed_down, w2_expert_stride_words, suh_down, suh2_stride, svh_down, svh2_stride, limit,
+                           out, workspace, workspace_bytes, stream);
 }
 
 extern "C" int exl3_moe_decode_noalloc(const uint16_t* x, int64_t tokens, int hidden, const void* topk_ids,

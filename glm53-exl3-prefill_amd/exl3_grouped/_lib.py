@@ -39,6 +39,7 @@ SIGNATURES = {
                                           P, P, P, P, P, P, I64, P]),
     "exl3_row_had": (I32, [P, P, P, P, P, I64, I64, I64, I32, I32, P]),
     "exl3_row_had_ex": (I32, [P, P, P, P, P, I64, I64, I64, I32, I32, I32, P]),
+    "exl3_row_had_gather_bf16": (I32, [P, P, P, P, P, I64, I64, I64, I32, P]),
     "exl3_act_had": (I32, [P, I64, P, P, P, I64, I64, I32, F32, P]),
     "exl3_act_had_ex": (I32, [P, I64, P, P, P, I64, I64, I32, F32, I32, P]),
     "exl3_act_had_f32": (I32, [P, I64, P, P, P, I64, I64, I32, F32, P]),
@@ -67,6 +68,8 @@ SIGNATURES = {
                                     P]),
     "exl3_moe_decode_workspace_bytes": (I64, [I64, I32, I32, I32, I32]),
     "exl3_moe_decode": (I32, [P, I64, I32, P, I32, P, I32, I32, I32, I32, I32, P, P, I64, P, I64, P, P, I64, P, I64,
+                              P, I64, P, I64, F32, P, P, I64, P]),
+    "exl3_moe_decode_dt": (I32, [P, I32, I64, I32, P, I32, P, I32, I32, I32, I32, I32, P, P, I64, P, I64, P, P, I64, P, I64,
                               P, I64, P, I64, F32, P, P, I64, P]),
     "exl3_moe_decode_noalloc": (I32, [P, I64, I32, P, I32, P, I32, I32, I32, I32, I32, P, P, I64, P, I64, P, P, I64,
                                       P, I64, P, I64, P, I64, F32, P, P]),

@@ -278,6 +278,26 @@ def row_had(src: torch.Tensor, dst: torch.Tensor, token_sorted: Optional[torch.T
                   _p(suh), suh.stride(0), suh.size(-1), rows, K, 1 if gather else 0, int(dst_layout), s)
 
 
+def row_had_gather_bf16(src: torch.Tensor, dst: torch.Tensor, token_sorted: torch.Tensor, expert_of_row: torch.Tensor,
+                        suh: torch.Tensor, rows: int) -> None:
+    """row_had(src.to(fp16), dst, ..., gather=True, dst_layout=1, rows=rows) for bf16 src [*, K], without the cast's pass
+    over it (new): each value is rounded to fp16 as it is read."""
+    K = dst.shape[1]
+    _check(dst.shape[0] >= t16_rows(rows), "T16 dst needs rows= and t16_rows(rows) rows")
+    _check(K % 128 == 0 and suh.size(-1) == K, "K must be a multiple of 128 and match suh")
+    _check(src.dtype == torch.bfloat16 and dst.dtype == torch.float16 and suh.dtype == torch.float16,
+           "bf16 src, fp16 dst and suh")
+    _check(src.dim() == 2 and src.size(1) == K and src.is_contiguous() and dst.is_contiguous(),
+           "src / dst must be contiguous [*, K]")
+    _check(suh.dim() == 2 and suh.stride(1) == 1, "suh must be [E, K] with unit inner stride")
+    _check(expert_of_row.dtype == torch.int32 and expert_of_row.numel() >= rows, "expert_of_row int32 [rows]")
+    _check(token_sorted.dtype == torch.int64 and token_sorted.numel() >= rows, "token_sorted int64 [rows]")
+    dev = _require_cuda(src, dst, expert_of_row, suh, token_sorted)
+    with _On(dev) as s:
+        _lib.call("exl3_row_had_gather_bf16", _p(src), _p(dst), _p(token_sorted), _p(expert_of_row), _p(suh),
+                  suh.stride(0), suh.size(-1), rows, K, s)
+
+
 def act_had(gu: torch.Tensor, act: torch.Tensor, expert_of_row: torch.Tensor, suh_down: torch.Tensor,
             limit: float, dst_layout: int = 0, gu_layout: int = 0, rows: Optional[int] = None) -> None:
     """kernel/exl3_grouped_prefill.cu:313-322. dst_layout (new): 0 row-major act [rows, I]; 1 T16 (rows = gu rows,
@@ -584,6 +604,18 @@ def moe_decode(x: torch.Tensor, topk_ids: torch.Tensor, topk_weights: torch.Tens
     [T, H]. One fixed launch sequence that allocates nothing when `out` and `workspace` (uint8, at least
     moe_decode_workspace_bytes(...) bytes, 256-byte aligned) are given, so the call can be captured in a graph."""
     _check(x.dim() == 2 and x.dtype == torch.float16 and x.is_contiguous(), "x must be contiguous fp16 [T, H]")
+    return moe_decode_dt(x, topk_ids, topk_weights, w13_trellis, w13_suh, w13_svh, w2_trellis, w2_suh, w2_svh, limit, out,
+                         workspace)
+
+
+def moe_decode_dt(x: torch.Tensor, topk_ids: torch.Tensor, topk_weights: torch.Tensor, w13_trellis: torch.Tensor,
+                  w13_suh: torch.Tensor, w13_svh: torch.Tensor, w2_trellis: torch.Tensor, w2_suh: torch.Tensor,
+                  w2_svh: torch.Tensor, limit: float, out: Optional[torch.Tensor] = None,
+                  workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """moe_decode for fp16 or bf16 x (new): bf16 values are rounded to fp16 as they are read, the result of
+    moe_decode(x.to(fp16), ...) without the cast's launch."""
+    _check(x.dim() == 2 and x.dtype in (torch.float16, torch.bfloat16) and x.is_contiguous(),
+           "x must be contiguous fp16 or bf16 [T, H]")
     T, H = x.shape
     _check(topk_ids.dim() == 2 and topk_ids.size(0) == T and topk_weights.shape == topk_ids.shape,
            "topk_ids / topk_weights must be [T, topk]")
@@ -622,7 +654,7 @@ def moe_decode(x: torch.Tensor, topk_ids: torch.Tensor, topk_weights: torch.Tens
     dev = _require_cuda(x, topk_ids, topk_weights, w13_trellis, w13_suh, w13_svh, w2_trellis, w2_suh, w2_svh, out,
                         workspace)
     with _On(dev) as s:
-        _lib.call("exl3_moe_decode", _p(x), T, H, _p(topk_ids), _DT[topk_ids.dtype], _p(topk_weights),
+        _lib.call("exl3_moe_decode_dt", _p(x), _DT[x.dtype], T, H, _p(topk_ids), _DT[topk_ids.dtype], _p(topk_weights),
                   _DT[topk_weights.dtype], topk, E, inter, bits, _p(g), _p(u), g.stride(0), _p(w13_suh[:, 0]),
                   w13_suh.stride(0), _p(w13_svh[:, 0]), _p(w13_svh[:, 1]), w13_svh.stride(0), _p(w2_trellis),
                   w2_trellis.stride(0), _p(w2_suh), w2_suh.stride(0), _p(w2_svh), w2_svh.stride(0), float(limit),

@@ -274,7 +274,9 @@ def grouped_prefill(x2d: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
     scatter = resolve_scatter(scatter, R)
     E = int(layer.w13_trellis.shape[0])
     I = int(layer._exl3_intermediate_local)
-    x16 = x2d.to(torch.float16).contiguous()
+    # bf16 rows are rounded to fp16 inside the input Hadamard; what it cannot read as it is gets cast in front
+    bf16 = x2d.dtype == torch.bfloat16 and x2d.is_contiguous() and x2d.data_ptr() % 16 == 0
+    xin = x2d if bf16 else x2d.to(torch.float16).contiguous()
     ids = ids.contiguous()
     weights = weights.contiguous()
     # row tiles of `tr` rows of one expert: each decoded trellis tile feeds up to `tr` rows of MFMA work
@@ -305,7 +307,10 @@ def grouped_prefill(x2d: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
         gp.build_tiles(counts, block_expert, block_row0, meta, tr)
         mark("build_blocks")
     h13 = B["h13"]
-    gp.row_had(x16, h13, token_sorted, expert_of_row, layer.w13_suh[:, 0], True, dst_layout=1, rows=R)
+    if bf16:
+        gp.row_had_gather_bf16(xin, h13, token_sorted, expert_of_row, layer.w13_suh[:, 0], R)
+    else:
+        gp.row_had(xin, h13, token_sorted, expert_of_row, layer.w13_suh[:, 0], True, dst_layout=1, rows=R)
     mark("row_had")
     gu = B["gu"]
     w13 = (layer.w13_trellis[:, 0], layer.w13_trellis[:, 1], layer.w13_svh[:, 0], layer.w13_svh[:, 1])
@@ -402,10 +407,13 @@ def moe_decode(x2d: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, laye
     E = int(layer.w13_trellis.shape[0])
     I = int(layer._exl3_intermediate_local)
     ws = reserve_decode_workspace(x2d.device, max(T, int(cap or 0)), topk, E, H, I)
-    x16 = x2d if x2d.dtype == torch.float16 and x2d.is_contiguous() else x2d.to(torch.float16).contiguous()
-    return gp.moe_decode(x16, ids.contiguous(), weights.contiguous(), layer.w13_trellis, layer.w13_suh,
-                         layer.w13_svh, layer.w2_trellis, layer.w2_suh, layer.w2_svh, float(limit), out=out,
-                         workspace=ws)
+    # bf16 rows are rounded to fp16 as the preparation reads them; what it cannot read as it is gets cast in front
+    as_is = x2d.is_contiguous() and (x2d.dtype == torch.float16 or
+                                     (x2d.dtype == torch.bfloat16 and x2d.data_ptr() % 16 == 0))
+    xin = x2d if as_is else x2d.to(torch.float16).contiguous()
+    return gp.moe_decode_dt(xin, ids.contiguous(), weights.contiguous(), layer.w13_trellis, layer.w13_suh,
+                            layer.w13_svh, layer.w2_trellis, layer.w2_suh, layer.w2_svh, float(limit), out=out,
+                            workspace=ws)
 
 
 def install(ov):

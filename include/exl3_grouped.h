@@ -165,6 +165,11 @@ int exl3_row_had(const uint16_t* src, uint16_t* dst, const int64_t* token_sorted
 int exl3_row_had_ex(const uint16_t* src, uint16_t* dst, const int64_t* token_sorted, const int32_t* expert_of_row,
                     const uint16_t* suh, int64_t suh_stride, int64_t suh_len, int64_t rows, int K, int gather,
                     int dst_layout, void* stream);
+/* exl3_row_had_ex(..., gather 1, EXL3_LAYOUT_T16) over bf16 src rows (bit patterns), each value rounded to fp16 first:
+ * the result of casting src to fp16 in front, without that pass over it. New. */
+int exl3_row_had_gather_bf16(const uint16_t* src, uint16_t* dst, const int64_t* token_sorted,
+                             const int32_t* expert_of_row, const uint16_t* suh, int64_t suh_stride, int64_t suh_len,
+                             int64_t rows, int K, void* stream);
 
 /*
  * Clamped SwiGLU + down Hadamard (pybind op act_had, kernel/exl3_grouped_prefill.cu:118-141 and :313-322):
@@ -385,6 +390,15 @@ int exl3_moe_decode(const uint16_t* x, int64_t tokens, int hidden, const void* t
                     int64_t svh13_stride, const uint16_t* packed_down, int64_t w2_expert_stride_words,
                     const uint16_t* suh_down, int64_t suh2_stride, const uint16_t* svh_down, int64_t svh2_stride,
                     float limit, float* out, void* workspace, int64_t workspace_bytes, void* stream);
+/* exl3_moe_decode with x in x_dtype (EXL3_DTYPE_F16, or EXL3_DTYPE_BF16: each value rounded to fp16 as it is read, the
+ * result of casting x in front). New. */
+int exl3_moe_decode_dt(const void* x, int x_dtype, int64_t tokens, int hidden, const void* topk_ids, int ids_dtype,
+                       const void* topk_weights, int weights_dtype, int topk, int n_experts, int inter, int bits,
+                       const uint16_t* packed_gate, const uint16_t* packed_up, int64_t w13_expert_stride_words,
+                       const uint16_t* suh_gate, int64_t suh13_stride, const uint16_t* svh_gate, const uint16_t* svh_up,
+                       int64_t svh13_stride, const uint16_t* packed_down, int64_t w2_expert_stride_words,
+                       const uint16_t* suh_down, int64_t suh2_stride, const uint16_t* svh_down, int64_t svh2_stride,
+                       float limit, float* out, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
  * exl3_moe_decode without a workspace argument: the workspace is a fixed 32 MiB scratch array in device memory that
