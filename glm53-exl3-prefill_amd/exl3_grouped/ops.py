@@ -14,7 +14,6 @@ workspace.
 """
 from __future__ import annotations
 
-import ctypes
 from typing import Optional
 
 import torch
@@ -31,33 +30,36 @@ def _check(cond: bool, msg: str) -> None:
 
 
 def _p(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def _require_cuda(*ts) -> torch.device:
-    for t in ts:
-        if t is not None:
-            _check(t.is_cuda, "tensors must be CUDA")
-    dev = next(t for t in ts if t is not None).device
-    for t in ts:
-        if t is not None:
-            _check(t.device == dev, "tensors must be on the same device")
-    return dev
+def _require_cuda(*ts) -> int:
+    """The index of the GPU all the tensors (None: not given) are on."""
+    at = [t.get_device() for t in ts if t is not None]         # -1: not on a GPU
+    _check(min(at) >= 0, "tensors must be CUDA")
+    _check(max(at) == min(at), "tensors must be on the same device")
+    return at[0]
 
 
 class _On:
-    """Device guard + current stream handle for one op call."""
+    """Device guard + current stream handle for one op call. The guard is only entered where the device is not the
+    current one already, and the handle is read without a Stream object around it: the two took 8 us of a call."""
 
-    def __init__(self, dev: torch.device):
+    __slots__ = ("dev", "guard")
+
+    def __init__(self, dev: int):
         self.dev = dev
+        self.guard = None
 
-    def __enter__(self):
-        self.guard = torch.cuda.device(self.dev)
-        self.guard.__enter__()
-        return ctypes.c_void_p(torch.cuda.current_stream(self.dev).cuda_stream)
+    def __enter__(self) -> int:
+        if torch.cuda.current_device() != self.dev:
+            self.guard = torch.cuda.device(self.dev)
+            self.guard.__enter__()
+        return torch._C._cuda_getCurrentRawStream(self.dev)
 
     def __exit__(self, *exc):
-        self.guard.__exit__(*exc)
+        if self.guard is not None:
+            self.guard.__exit__(*exc)
         return False
 
 
@@ -623,42 +625,42 @@ def moe_decode_dt(x: torch.Tensor, topk_ids: torch.Tensor, topk_weights: torch.T
     _check(topk_weights.dtype in (torch.float32, torch.float16, torch.bfloat16) and topk_weights.is_contiguous(),
            "topk_weights fp32/fp16/bf16")
     topk = topk_ids.size(1)
-    _check(w13_trellis.dim() == 5 and w13_trellis.size(1) == 2 and w13_trellis.dtype in (torch.int16, torch.uint16),
+    # the gate and up halves are addressed by their offsets: a view of each per call costs as much as a launch
+    s13 = tuple(w13_trellis.shape)
+    _check(len(s13) == 5 and s13[1] == 2 and w13_trellis.dtype in (torch.int16, torch.uint16),
            "w13_trellis must be [E, 2, H/16, I/16, 16*bits] int16")
-    E = w13_trellis.size(0)
-    words = w13_trellis.size(4)
+    E, words = s13[0], s13[4]
     _check(words in (32, 48, 64), "trellis tile width must be 16*bits words, bits in {2, 3, 4}")
     bits = words // 16
-    _check(w13_trellis.size(2) * 16 == H, "w13_trellis K must match x")
-    inter = w13_trellis.size(3) * 16
-    g, u = w13_trellis[:, 0], w13_trellis[:, 1]
-    for t in (g, u):
-        _check(t.stride(3) == 1 and t.stride(2) == words and t.stride(1) == t.size(2) * words,
-               "w13_trellis inner dims must be contiguous")
-    _check(w2_trellis.dim() == 4 and w2_trellis.shape == (E, inter // 16, H // 16, words) and
-           w2_trellis.dtype == w13_trellis.dtype and w2_trellis.stride(3) == 1 and w2_trellis.stride(2) == words and
-           w2_trellis.stride(1) == w2_trellis.size(2) * words, "w2_trellis must be [E, I/16, H/16, 16*bits]")
-    _check(w13_suh.shape == (E, 2, H) and w13_svh.shape == (E, 2, inter) and w2_suh.shape == (E, inter) and
-           w2_svh.shape == (E, H), "sign / scale vector shapes")
+    _check(s13[2] * 16 == H, "w13_trellis K must match x")
+    inter = s13[3] * 16
+    st13 = w13_trellis.stride()
+    _check(st13[4] == 1 and st13[3] == words and st13[2] == s13[3] * words, "w13_trellis inner dims must be contiguous")
+    st2 = w2_trellis.stride()
+    _check(len(st2) == 4 and tuple(w2_trellis.shape) == (E, inter // 16, H // 16, words) and
+           w2_trellis.dtype == w13_trellis.dtype and st2[3] == 1 and st2[2] == words and st2[1] == H // 16 * words,
+           "w2_trellis must be [E, I/16, H/16, 16*bits]")
+    _check(tuple(w13_suh.shape) == (E, 2, H) and tuple(w13_svh.shape) == (E, 2, inter) and
+           tuple(w2_suh.shape) == (E, inter) and tuple(w2_svh.shape) == (E, H), "sign / scale vector shapes")
     for t in (w13_suh, w13_svh, w2_suh, w2_svh):
         _check(t.dtype == torch.float16 and t.stride(-1) == 1, "suh / svh must be fp16 with contiguous rows")
-    _check(w13_svh[:, 0].stride() == w13_svh[:, 1].stride(), "gate / up svh strides must match")
     if out is None:
         out = torch.empty(T, H, dtype=torch.float32, device=x.device)
     _check(out.dtype == torch.float32 and tuple(out.shape) == (T, H) and out.is_contiguous(), "out must be fp32 [T, H]")
     need = moe_decode_workspace_bytes(T, topk, E, H, inter)
     if workspace is None:
         workspace = torch.empty(max(need, 256), dtype=torch.uint8, device=x.device)
-    _check(workspace.is_contiguous() and workspace.numel() * workspace.element_size() >= need,
-           "decode workspace too small")
+    ws_bytes = workspace.numel() * workspace.element_size()
+    _check(workspace.is_contiguous() and ws_bytes >= need, "decode workspace too small")
     dev = _require_cuda(x, topk_ids, topk_weights, w13_trellis, w13_suh, w13_svh, w2_trellis, w2_suh, w2_svh, out,
                         workspace)
+    gate, svh_gate = w13_trellis.data_ptr(), w13_svh.data_ptr()
     with _On(dev) as s:
-        _lib.call("exl3_moe_decode_dt", _p(x), _DT[x.dtype], T, H, _p(topk_ids), _DT[topk_ids.dtype], _p(topk_weights),
-                  _DT[topk_weights.dtype], topk, E, inter, bits, _p(g), _p(u), g.stride(0), _p(w13_suh[:, 0]),
-                  w13_suh.stride(0), _p(w13_svh[:, 0]), _p(w13_svh[:, 1]), w13_svh.stride(0), _p(w2_trellis),
-                  w2_trellis.stride(0), _p(w2_suh), w2_suh.stride(0), _p(w2_svh), w2_svh.stride(0), float(limit),
-                  _p(out), _p(workspace), workspace.numel() * workspace.element_size(), s)
+        _lib.call("exl3_moe_decode_dt", x.data_ptr(), _DT[x.dtype], T, H, topk_ids.data_ptr(), _DT[topk_ids.dtype],
+                  topk_weights.data_ptr(), _DT[topk_weights.dtype], topk, E, inter, bits, gate, gate + 2 * st13[1],
+                  st13[0], w13_suh.data_ptr(), w13_suh.stride(0), svh_gate, svh_gate + 2 * w13_svh.stride(1),
+                  w13_svh.stride(0), w2_trellis.data_ptr(), st2[0], w2_suh.data_ptr(), w2_suh.stride(0),
+                  w2_svh.data_ptr(), w2_svh.stride(0), float(limit), out.data_ptr(), workspace.data_ptr(), ws_bytes, s)
     return out
 
 
