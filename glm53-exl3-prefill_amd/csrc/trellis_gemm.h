@@ -1063,6 +1063,22 @@ __device__ __forceinline__ void thin_mainloop(const GemmParams& p, const Tile& t
     if (s0 < num_kb) trip(s0, std::integral_constant<int, 2>{});   // num_kb is even
 }
 
+// A row group's accumulators of wave w's 32 columns into LDS, in the layout of the shared epilogue (column block nb's
+// floatx4 of lane l at xs[64 nb + l]): n-tile 2 w's columns 4 kq .. + 3 are x of lane groups 0, 1 then y of 0, 1; n-tile
+// 2 w + 1's those of 2, 3.
+__device__ __forceinline__ void hand_over_group(floatx4 (&a)[2], floatx4* xs, int wave, int lane)
+{
+    #pragma unroll
+    for (int r = 0; r < 4; ++r)
+    {
+        const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[0][r]), __float_as_uint(a[1][r]), false, false);
+        a[0][r] = __uint_as_float(v[0]);
+        a[1][r] = __uint_as_float(v[1]);
+    }
+    xs[(2 * wave) * 64 + lane] = a[0];
+    xs[(2 * wave + 1) * 64 + lane] = a[1];
+}
+
 // A thin tile of at most GROUPS row groups: the main loop, then the epilogue, four row groups (one per wave) at a time.
 template <int BITS, int MODE, int GROUPS, bool ACT_IN, bool NT>
 __device__ __forceinline__ void thin_groups(const GemmParams& p, const Tile& t, int group, int wave, int lane,
@@ -1079,25 +1095,10 @@ __device__ __forceinline__ void thin_groups(const GemmParams& p, const Tile& t, 
 
     floatx4* xs = reinterpret_cast<floatx4*>(lds_raw);
     float* const stage = reinterpret_cast<float*>(lds_raw) + wave * (16 * SC_ROW);
-    // row groups g0 .. g0 + 3 into LDS, in the layout of the shared epilogue: n-tile 2 w's columns 4 kq .. + 3 are x of lane
-    // groups 0, 1 then y of 0, 1; n-tile 2 w + 1's those of 2, 3
-    auto hand_over = [&](auto g0_tag) {
+    auto hand_over = [&](auto g0_tag) {                            // row groups g0 .. g0 + 3
         constexpr int G0 = decltype(g0_tag)::value;
         #pragma unroll
-        for (int i = 0; i < 4 && G0 + i < GROUPS; ++i)
-        {
-            floatx4 (&a)[2] = acc[G0 + i];
-            #pragma unroll
-            for (int r = 0; r < 4; ++r)
-            {
-                const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[0][r]), __float_as_uint(a[1][r]), false,
-                                                                false);
-                a[0][r] = __uint_as_float(v[0]);
-                a[1][r] = __uint_as_float(v[1]);
-            }
-            xs[(8 * i + 2 * wave) * 64 + lane] = a[0];
-            xs[(8 * i + 2 * wave + 1) * 64 + lane] = a[1];
-        }
+        for (int i = 0; i < 4 && G0 + i < GROUPS; ++i) hand_over_group(acc[G0 + i], xs + 8 * i * 64, wave, lane);
     };
     __syncthreads();                                               // the activations are dead
     hand_over(std::integral_constant<int, 0>{});
@@ -1425,6 +1426,75 @@ int launch_gemm_kpair(const GemmParams& p, hipStream_t s)
     return fail("internal: K-pair launch for mode %d", MODE);
 }
 
+// A dense GEMM of so few rows that its 64-row tiles leave CUs idle (a small decode batch's projection: 32 workgroups for 4096
+// columns) lasts as long as one workgroup's whole K range: latency, at one wave per SIMD. Here one workgroup of 16 waves
+// takes the tile, KSLICES groups of four waves over equal parts of K, each the thin main loop with its own activation
+// chunks (the barriers are shared: all run the same stages); the partial sums are then added through LDS in slice order,
+// so the result is the same on every run, and the first group's waves run the epilogue. A linear of 7 x 4096 x 4096 with
+// its input Hadamard: 33.0 -> 26.2 us per call.
+constexpr int KSLICES = 4;
+
+template <int BITS, int MODE, int GROUPS>
+__device__ __forceinline__ void kslice_groups(const GemmParams& p, const Tile& t, int wave16, int lane,
+                                              unsigned char* lds_raw)
+{
+    const int slice = wave16 >> 2, wave = wave16 & 3;
+    Tile part = t;
+    part.num_kb = t.num_kb / KSLICES;                              // even: the host requires K % (64 KSLICES) == 0
+    part.kb0 = t.kb0 + slice * part.num_kb;
+    floatx4 acc[GROUPS][2];
+    #pragma unroll
+    for (int g = 0; g < GROUPS; ++g) acc[g][0] = acc[g][1] = floatx4{};
+    floatx4* const xs = reinterpret_cast<floatx4*>(lds_raw + slice * THIN_LDS_BYTES);
+    thin_mainloop<BITS, MODE, GROUPS, false, false>(p, part, wave, lane, reinterpret_cast<uint4*>(xs), acc);
+    __syncthreads();                                               // the activations are dead
+    #pragma unroll
+    for (int g = 0; g < GROUPS; ++g) hand_over_group(acc[g], xs + 8 * g * 64, wave, lane);
+    __syncthreads();
+    const int n_groups = (t.rows_valid + 15) >> 4;
+    if (slice != 0 || wave >= n_groups) return;
+    floatx4 full[1][8];
+    #pragma unroll
+    for (int nb = 0; nb < 8; ++nb)
+    {
+        full[0][nb] = xs[(8 * wave + nb) * 64 + lane];
+        #pragma unroll
+        for (int s = 1; s < KSLICES; ++s) full[0][nb] += xs[s * (THIN_LDS_BYTES / 16) + (8 * wave + nb) * 64 + lane];
+    }
+    epilogue<MODE, 1, 0>(p, t, wave, lane, full, nullptr);
+}
+
+template <int BITS, int MODE>
+__global__ __launch_bounds__(256 * KSLICES, 4)
+void trellis_gemm_kslice_kernel(const GemmParams p)
+{
+    static_assert(MODE == MODE_STORE_F32 || MODE == MODE_STORE_F16, "plain-store modes");
+    __shared__ __align__(16) unsigned char lds_raw[KSLICES * THIN_LDS_BYTES];
+    int group, slot;
+    xcd_group_slot((int) blockIdx.x, p.n_slots, group, slot);
+    Tile t;
+    if (!resolve_tile<true>(p, group, slot, t)) return;           // uniform over the workgroup
+    const int lane = threadIdx.x & 63;
+    const int wave16 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n_groups = (t.rows_valid + 15) >> 4;                 // uniform
+    if (n_groups == 1) kslice_groups<BITS, MODE, 1>(p, t, wave16, lane, lds_raw);
+    else if (n_groups == 2) kslice_groups<BITS, MODE, 2>(p, t, wave16, lane, lds_raw);
+    else kslice_groups<BITS, MODE, 4>(p, t, wave16, lane, lds_raw);
+}
+
+// The K-slice schedule for a dense store: 64-row tiles, one 16-wave workgroup per (tile, 128-column block).
+template <int BITS, int MODE>
+int launch_gemm_kslice(const GemmParams& p, hipStream_t s)
+{
+    if (p.tile_rows != 64 || p.size_k % (64 * KSLICES) != 0 || p.k_split > 1)
+        return fail("internal: K-slice launch needs 64-row tiles and K %% %d == 0", 64 * KSLICES);
+    const int64_t grid = (int64_t) (p.n_groups + 7) / 8 * 8 * p.n_slots;
+    if (grid == 0) return EXL3_OK;
+    if (grid > 0x7FFFFFFF) return fail("grid too large");
+    trellis_gemm_kslice_kernel<BITS, MODE><<<(unsigned) grid, 256 * KSLICES, 0, s>>>(p);
+    return EXL3_OK;
+}
+
 // 512-row tiles run the 8-wave variant, 256-row tiles the 4-wave kernel, 64- and 128-row tiles the thin one, which
 // decodes a tile's weights with half the instructions' waiting and no LDS traffic for them: 288 tiles of 72 / 96 / 128
 // rows, gate|up 547 / 648 / 676 us on the 4-wave kernel against 504 / 508 / 573, down 373 / 414 / 456 against 331 / 350 /
@@ -1475,6 +1545,9 @@ int launch_gemm_b4d(int mode, const GemmParams& p, hipStream_t s);
 int launch_gemm_kpair_b2(int mode, const GemmParams& p, hipStream_t s);
 int launch_gemm_kpair_b3(int mode, const GemmParams& p, hipStream_t s);
 int launch_gemm_kpair_b4(int mode, const GemmParams& p, hipStream_t s);
+int launch_gemm_kslice_b2(int mode, const GemmParams& p, hipStream_t s);
+int launch_gemm_kslice_b3(int mode, const GemmParams& p, hipStream_t s);
+int launch_gemm_kslice_b4(int mode, const GemmParams& p, hipStream_t s);
 int launch_gemm_actin_b2(const GemmParams& p, hipStream_t s);
 int launch_gemm_actin_b3(const GemmParams& p, hipStream_t s);
 int launch_gemm_actin_b4(const GemmParams& p, hipStream_t s);

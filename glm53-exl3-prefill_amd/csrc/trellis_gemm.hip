@@ -218,6 +218,20 @@ int launch_kpair_bits(int bits, GemmParams p, hipStream_t s)
     }
 }
 
+// The K-slice schedule (trellis_gemm_kslice_kernel): a dense store on 64-row tiles, four K slices of a tile in one 16-wave
+// workgroup.
+template <int MODE>
+int launch_kslice_bits(int bits, const GemmParams& p, hipStream_t s)
+{
+    switch (bits)
+    {
+        case 2: return launch_gemm_kslice_b2(MODE, p, s);
+        case 3: return launch_gemm_kslice_b3(MODE, p, s);
+        case 4: return launch_gemm_kslice_b4(MODE, p, s);
+        default: return fail("unsupported bits %d (2, 3 or 4)", bits);
+    }
+}
+
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 
 }  // namespace
@@ -520,6 +534,19 @@ bool dense_kpair_pays(int64_t m, int n_slots, int size_k)
     return dense_split_pays(m, n_slots, size_k) && (m + 255) / 256 * n_slots * 10 >= 7 * device_cus();
 }
 
+// The dense linear on 64-row tiles runs the K-slice schedule while its workgroups fit one per CU (it takes a CU's whole
+// LDS; a second round of 16-wave workgroups would cost a whole K range more). An fp32 output of fewer than 32 tiles keeps
+// the two slices on CUs of their own (dense_split_pays): with its input Hadamard, fp16 / fp32 us per call, before -> here:
+// 7 x 4096 x 4096 33.6 / 30.4 -> 27.1 / 26.8, 64 rows 43.3 / 39.5 -> 35.2 / 35.5, 250 rows 44.8 / 42.9 -> 37.2 / 37.2
+// (32 and 128 tiles); 7 x 4096 x 1536 at 3 bits 34.7 / 23.1 -> 27.7 / 27.2, 40 x 2048 x 2048 at 2 bits 24.1 / 18.3 ->
+// 22.1 / 21.9 (12 and 16 tiles). (The fat GEMM keeps its schedules: all its variants sum K in one order.)
+bool dense_kslice_pays(const GemmParams& p, bool f32)
+{
+    const int64_t tiles = (int64_t) p.n_groups * p.n_slots;
+    return p.tile_rows == 64 && p.size_k % (64 * KSLICES) == 0 && tiles <= device_cus() &&
+           (!f32 || tiles >= 32 || !dense_split_pays(p.m, p.n_slots, p.size_k));
+}
+
 template <int MODE>
 int launch_dense_split2(GemmParams p, int bits, float* out, int64_t out_floats, hipStream_t s, int variant = 1)
 {
@@ -613,7 +640,10 @@ extern "C" int exl3_linear(const uint16_t* x, int64_t m, int k, const uint16_t* 
     p.a = work; p.a_rows = m; p.a_t16 = 1; p.size_k = k; p.packed0 = packed; p.tiles_n = tiles_n;
     p.svh0 = svh; p.tile_rows = dense_tile_rows(m, k); p.n_groups = (int) ((m + p.tile_rows - 1) / p.tile_rows);
     p.n_tiles_each = n / TILE_N; p.n_slots = p.n_tiles_each; p.m = m; p.out = out; p.out_ld = n;
-    if (dense_kpair_pays(m, p.n_slots, k))
+    if (dense_kslice_pays(p, out_dtype == EXL3_DTYPE_F32))
+        rc = out_dtype == EXL3_DTYPE_F32 ? launch_kslice_bits<MODE_STORE_F32>(bits, p, s)
+                                         : launch_kslice_bits<MODE_STORE_F16>(bits, p, s);
+    else if (dense_kpair_pays(m, p.n_slots, k))
         rc = out_dtype == EXL3_DTYPE_F32 ? launch_kpair_bits<MODE_STORE_F32>(bits, p, s)
                                          : launch_kpair_bits<MODE_STORE_F16>(bits, p, s);
     else if (out_dtype == EXL3_DTYPE_F32 && dense_split_pays(m, p.n_slots, k))

@@ -26,6 +26,17 @@ int launch_gemm_b3(int mode, bool dense, const GemmParams& p, hipStream_t s)
     return fail("internal: no kernel for mode %d", mode);
 }
 
+int launch_gemm_kslice_b3(int mode, const GemmParams& p, hipStream_t s)
+{
+    switch (mode)
+    {
+        case MODE_STORE_F16: return launch_gemm_kslice<3, MODE_STORE_F16>(p, s);
+        case MODE_STORE_F32: return launch_gemm_kslice<3, MODE_STORE_F32>(p, s);
+        default: break;
+    }
+    return fail("internal: no K-slice kernel for mode %d", mode);
+}
+
 int launch_gemm_kpair_b3(int mode, const GemmParams& p, hipStream_t s)
 {
     switch (mode)

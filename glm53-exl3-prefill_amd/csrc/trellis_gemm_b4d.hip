@@ -16,6 +16,17 @@ int launch_gemm_b4d(int mode, const GemmParams& p, hipStream_t s)
     return fail("internal: no kernel for mode %d", mode);
 }
 
+int launch_gemm_kslice_b4(int mode, const GemmParams& p, hipStream_t s)
+{
+    switch (mode)
+    {
+        case MODE_STORE_F16: return launch_gemm_kslice<4, MODE_STORE_F16>(p, s);
+        case MODE_STORE_F32: return launch_gemm_kslice<4, MODE_STORE_F32>(p, s);
+        default: break;
+    }
+    return fail("internal: no K-slice kernel for mode %d", mode);
+}
+
 int launch_gemm_kpair_b4(int mode, const GemmParams& p, hipStream_t s)
 {
     switch (mode)
