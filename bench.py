@@ -12,8 +12,8 @@ collection inside the timed steps would stall the launching thread for 30-40 ms.
 
 Prints ONE JSON line: value = routed tokens/s (T*topk / step time); ms_per_step = per-layer MoE ms; stage_ms = the
 median over the timed steps of each stage's HIP-event time on the launch stream (stage_ms_mean beside it); roofline of
-the dominant stage (the gate|up grouped GEMM: full expert tiles on the main kernel, each expert's last tile of <= 64
-rows on the thin kernel; MFMA-bound: algorithmic 4*R*H*I flop per stage call over its median duration) and
+the dominant stage (the gate|up grouped GEMM: full expert tiles on the main kernel, each expert's small last
+tile on the thin kernel; MFMA-bound: algorithmic 4*R*H*I flop per stage call over its median duration) and
 roofline_down for the down GEMM and its output stages (2*R*H*I flop). From the committed rocprofv3 summaries of the same workload
 (profiles/grouped_prefill_headline_*.md): traffic (calibrated FETCH_SIZE + WRITE_SIZE bytes per stage call),
 stage_hbm_gbs (those bytes over this run's stage time) and counters (matrix-pipe and VALU busy fractions from
@@ -46,20 +46,20 @@ REFERENCE_GB10_MS = {1024: 11.4, 2048: 13.7, 4096: 20.2, 8192: 33.2}
 HBM_PEAK_GBS = 8000.0
 # The kernels of each stage of grouped_prefill as rocprofv3 names them (namespaces and parameter lists stripped; the keys
 # of the committed profile summaries): the GEMMs run full expert tiles on the main kernel and each expert's last tile
-# of <= 64 rows on the thin one.
+# of at most 64 (128 where such tiles are many) rows on the thin one.
 STAGE_KERNELS = {
     "sort_routes": ("sort_hist_kernel", "sort_scatter_tiles_kernel"),         # + the tile tables
     "row_had": ("row_had_t16_kernel<true>",),
-    "gemm_gate_up": ("trellis_gemm_kernel<{bits}, 0, false, 4, 4, false>", "trellis_gemm_kernel<{bits}, 0, false, 1, 4, true>"),
+    "gemm_gate_up": ("trellis_gemm_kernel<{bits}, 0, false, 4, 4, false>", "trellis_gemm_kernel<{bits}, 0, false, 2, 4, true>"),
     "act_had": ("act_had_t16_kernel<false, true>",),
 }
 # The down projection's stages by output method: the fp32 atomic scatter by token (mode 1), or per-route fp32 rows
 # (mode 2) and their fixed-order sum per token.
 DOWN_STAGE_KERNELS = {
     "atomic": {"gemm_down_scatter": ("trellis_gemm_kernel<{bits}, 1, false, 4, 4, false>",
-                                     "trellis_gemm_kernel<{bits}, 1, false, 1, 4, false>")},
+                                     "trellis_gemm_kernel<{bits}, 1, false, 2, 4, false>")},
     "combine": {"gemm_down_routes": ("trellis_gemm_kernel<{bits}, 3, false, 4, 4, false>",
-                                     "trellis_gemm_kernel<{bits}, 3, false, 1, 4, true>"),
+                                     "trellis_gemm_kernel<{bits}, 3, false, 2, 4, true>"),
                 "combine": ("combine_routes_cols_kernel<8, 0>",)},
 }
 
