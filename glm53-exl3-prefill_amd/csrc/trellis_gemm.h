@@ -150,10 +150,17 @@ __device__ __forceinline__ void fwht32(float (&x)[32])
             }
 }
 
-// Raw stream dwords a lane holds per stage. K=4 / K=2: the lane's own 2 / 1 dwords of the tile (one coalesced load
-// per 16-lane row) -- the 16-bit look-back of its first chunk is the previous lane's last dword (DPP rotate);
-// K=3: the three dwords its two windows touch, loaded directly.
-template <int BITS> constexpr int raw_words() { return BITS == 4 ? 2 : (BITS == 2 ? 1 : 3); }
+// Raw stream dwords a lane holds per stage for the chunk pair 2 j, 2 j + 1 of a tile (one coalesced load per 16-lane row): its
+// own 2 / 1 dwords at 4 / 2 bits; at 3 bits (where loading all three dwords of both windows took three loads: a 2500-token
+// layer call 1122 -> 1107 us) pairs 2 a and 2 a + 1 share the dwords 3 a .. + 2, the even pair holding the
+// first two, the odd one the last two. The look-back before them (4 and 2 bits: 16 bits of every pair's first chunk; 3
+// bits: the even pair's) is the last dword of the lane with the previous pair.
+template <int BITS> constexpr int raw_words() { return BITS == 2 ? 1 : 2; }
+// Dword of the tile at which pair j's own words start.
+template <int BITS> __device__ __forceinline__ int raw_start(int j)
+{
+    return BITS == 3 ? 3 * (j >> 1) + (j & 1) : raw_words<BITS>() * j;
+}
 
 // Value of `v` in the previous lane of this lane's 16-lane row (lane 0 of the row gets lane 15's).
 __device__ __forceinline__ uint32_t prev_in_row(uint32_t v)
@@ -237,8 +244,8 @@ __device__ __forceinline__ bool resolve_tile(const GemmParams& p, int group, int
 // a = j16 >> 1 and a + 8, rows 4 b .. 4 b + 3 and 8 + 4 b .. with b = j16 & 1.
 template <int N> struct Chunks { Chunk4 c[N]; };
 
-// Chunks 2 j and 2 j + 1 of a tile (positions 16 j .. + 15): from the tile's dwords 2 j, 2 j + 1 (4 bits) or dword j (2
-// bits) in r with the dword before them in prev, or from the three dwords the two windows touch (3 bits; odd = j & 1).
+// Chunks 2 j and 2 j + 1 of a tile (positions 16 j .. + 15) from the pair's own words r and the dword before them; odd =
+// j & 1.
 template <int BITS>
 __device__ __forceinline__ void decode_pair(uint32_t prev, const uint32_t (&r)[raw_words<BITS>()], int odd, Chunks<2>& o)
 {
@@ -254,12 +261,12 @@ __device__ __forceinline__ void decode_pair(uint32_t prev, const uint32_t (&r)[r
     }
     else
     {
-        // The windows start 19 / 43 bits (j even) or 3 / 27 bits (odd) into r[0]. Even ones shift their words down by
-        // 16 bits first, so both kinds decode at the compile-time offsets 3 and 27: constant shifts of a 64-bit window
-        // compile to 32-bit funnel shifts, while per-lane 64-bit shift amounts feeding the decoder's asm gave wrong
+        // The windows start 3 / 27 bits into an odd pair's words, and 16 bits before an even pair's, which are funnelled
+        // into place first, so both kinds decode at the compile-time offsets 3 and 27: constant shifts of a 64-bit
+        // window compile to 32-bit funnel shifts, while per-lane 64-bit shift amounts feeding the decoder's asm gave wrong
         // results at random.
-        const uint32_t x0 = odd ? r[0] : __builtin_amdgcn_alignbit(r[1], r[0], 16);
-        const uint32_t x1 = odd ? r[1] : __builtin_amdgcn_alignbit(r[2], r[1], 16);
+        const uint32_t x0 = odd ? r[0] : __builtin_amdgcn_alignbit(r[0], prev, 16);
+        const uint32_t x1 = odd ? r[1] : __builtin_amdgcn_alignbit(r[1], r[0], 16);
         o.c[0] = decode_chunk<3, 3>(x0, x1);
         o.c[1] = decode_chunk<3, 27>(x0, x1);
     }
@@ -273,7 +280,7 @@ struct Decoder
     using Out = Chunks<2>;
     __amdgpu_buffer_rsrc_t raw;    // based at the wave's first tile of stage 0
     int stage_bytes, last_kb, tb, wcol0, wcol1;
-    uint32_t off[NR];              // per-lane byte offsets of the raw words
+    uint32_t off;                  // per-lane byte offset of the raw words
 
     __device__ __forceinline__ Decoder(const GemmParams& p, const Tile& t, int dw, int lane, int num_kb)
     {
@@ -287,17 +294,7 @@ struct Decoder
         raw = buffer_rsrc(t.packed + first, ((int64_t) (p.size_k >> 4) * p.tiles_n * NDW - first) * 4);
         last_kb = num_kb - 1;
         const int tile_off = (lane >> 4) * NDW;
-        if constexpr (BITS == 3)
-        {
-            const int d0 = (16 * j16 * BITS + BITS - 16) >> 5;  // dword of the first window bit (may be -1)
-            #pragma unroll
-            for (int i = 0; i < NR; ++i) off[i] = 4 * (tile_off + (d0 + i + NDW) % NDW);
-        }
-        else
-        {
-            #pragma unroll
-            for (int i = 0; i < NR; ++i) off[i] = 4 * (tile_off + NR * j16 + i);
-        }
+        off = 4 * (tile_off + raw_start<BITS>(j16));
         wcol0 = nt8 * LDS_BLK + ta * LDS_ROW + kt * 16 + 4 * tb;         // column a, rows 4 b ..
         wcol1 = wcol0 + 8 * LDS_ROW;                                    // column a + 8
     }
@@ -305,22 +302,18 @@ struct Decoder
     __device__ __forceinline__ void load(int kb, uint32_t (&r)[NR]) const
     {
         const int so = min(kb, last_kb) * stage_bytes;
-        if constexpr (BITS == 4)
+        if constexpr (NR == 2)
         {
-            const auto v = __builtin_amdgcn_raw_buffer_load_b64(raw, off[0], so, 0);
+            const auto v = __builtin_amdgcn_raw_buffer_load_b64(raw, off, so, 0);
             r[0] = v[0];
             r[1] = v[1];
         }
         else
-        {
-            #pragma unroll
-            for (int i = 0; i < NR; ++i) r[i] = __builtin_amdgcn_raw_buffer_load_b32(raw, off[i], so, 0);
-        }
+            r[0] = __builtin_amdgcn_raw_buffer_load_b32(raw, off, so, 0);
     }
     __device__ __forceinline__ void decode(const uint32_t (&r)[NR], Out& o) const
     {
-        if constexpr (BITS == 3) decode_pair<3>(0u, r, tb, o);
-        else decode_pair<BITS>(prev_in_row(r[NR - 1]), r, tb, o);
+        decode_pair<BITS>(prev_in_row(r[NR - 1]), r, tb, o);
     }
     __device__ __forceinline__ void store(const Out& o, uint16_t* lds) const
     {
@@ -409,7 +402,7 @@ struct ColDecoder
 {
     static constexpr int AUX = NT ? 2 : 0;                // buffer-load cache policy: 2 = non-temporal
     static constexpr int NDW = 8 * BITS;                  // dwords per tile
-    static constexpr int NR = BITS == 2 ? 1 : 2;
+    static constexpr int NR = raw_words<BITS>();
     __amdgpu_buffer_rsrc_t raw;    // based at the wave's first tile of stage 0
     int stage_bytes, last_kb, odd;
     uint32_t off;                  // per-lane byte offset of the own words
@@ -424,10 +417,7 @@ struct ColDecoder
         const int64_t first = ((int64_t) (2 * t.kb0) * p.tiles_n + t.nt * 8 + 2 * wave) * NDW;
         raw = buffer_rsrc(t.packed + first, ((int64_t) (p.size_k >> 4) * p.tiles_n * NDW - first) * 4);
         last_kb = num_kb - 1;
-        // 3 bits: pairs 2 a and 2 a + 1 share the dwords 3 a .. + 2, the even one owns the first two (its window starts in
-        // the dword before them), the odd one the last two (its window lies inside)
-        const int d = BITS == 3 ? 3 * (i & 7) + odd : NR * j;
-        off = 4 * (((q >> 1) * p.tiles_n + (i >> 3)) * NDW + d);
+        off = 4 * (((q >> 1) * p.tiles_n + (i >> 3)) * NDW + raw_start<BITS>(j));
         const int jp = (j + 15) & 15;
         before = 4 * (16 * ((q & 2) | (jp & 1)) + (i & 8) + (jp >> 1));
     }
@@ -451,13 +441,7 @@ struct ColDecoder
     {
         typedef uint32_t u4 __attribute__((ext_vector_type(4)));
         Chunks<2> o;
-        if constexpr (BITS == 3)
-        {
-            const uint32_t w[3] = {odd ? r[0] : prev, odd ? r[1] : r[0], r[1]};
-            decode_pair<3>(0u, w, odd, o);
-        }
-        else
-            decode_pair<BITS>(prev, r, odd, o);
+        decode_pair<BITS>(prev, r, odd, o);
         auto natural = [](uint32_t& first, uint32_t& second) {
             const auto v = __builtin_amdgcn_permlane16_swap(first, second, false, false);
             first = v[0];
