@@ -534,17 +534,25 @@ bool dense_kpair_pays(int64_t m, int n_slots, int size_k)
     return dense_split_pays(m, n_slots, size_k) && (m + 255) / 256 * n_slots * 10 >= 7 * device_cus();
 }
 
-// The dense linear on 64-row tiles runs the K-slice schedule while its workgroups fit one per CU (it takes a CU's whole
-// LDS; a second round of 16-wave workgroups would cost a whole K range more). An fp32 output of fewer than 32 tiles keeps
-// the two slices on CUs of their own (dense_split_pays): with its input Hadamard, fp16 / fp32 us per call, before -> here:
-// 7 x 4096 x 4096 33.6 / 30.4 -> 27.1 / 26.8, 64 rows 43.3 / 39.5 -> 35.2 / 35.5, 250 rows 44.8 / 42.9 -> 37.2 / 37.2
-// (32 and 128 tiles); 7 x 4096 x 1536 at 3 bits 34.7 / 23.1 -> 27.7 / 27.2, 40 x 2048 x 2048 at 2 bits 24.1 / 18.3 ->
-// 22.1 / 21.9 (12 and 16 tiles). (The fat GEMM keeps its schedules: all its variants sum K in one order.)
+// Whether the dense linear runs the K-slice schedule: 64-row tiles while the workgroups of the busiest XCD (a row group's
+// column tiles all run on one, xcd_group_slot) fit one per CU: with 128 of its 160 KB of LDS taken a CU holds one, where
+// the plain launch keeps four resident. Shorter K does not pay for handing the partial sums over, and an fp32 output
+// whose two slices (dense_split_pays) fit one workgroup per CU on that XCD keeps them. From K = 6144 two rounds still
+// pay against the plain launch. us per call with its input Hadamard, each call another matrix, 4 bits, plain (two slices)
+// / K slices at 7 and 64 rows:
+//   fp16, K x N: 512 x 4096 9.6 / 10.2, 12.6 / 13.3; 768 x 4096 11.3 / 11.4, 14.7 / 15.2; 1024 x 4096 13.0 / 12.6,
+//   16.9 / 16.6; 4096 x 4096 33.5 / 26.8, 43.6 / 34.7; 1024 x 4608 (36 tiles) 17.4 / 21.1, 23.1 / 27.7; 4096 x 8192
+//   47.3 / 48.8, 64.9 / 64.3; 6144 x 8192 67.2 / 66.2, 92.5 / 87.7; 6144 x 16384 117 / 129, 154 / 170;
+//   fp32: 4096 x 2048 (16 tiles) 21.9 / 25.6, 28.3 / 34.1; 4096 x 2304 28.9 / 25.6, 38.6 / 34.4.
+// The K-pair schedule is for taller tiles only: 4096 x 23040 at 7 and 64 rows 183 and 300 us, plain 114 and 152.
+// (The fat GEMM keeps its schedules: all its variants sum K in one order.)
 bool dense_kslice_pays(const GemmParams& p, bool f32)
 {
-    const int64_t tiles = (int64_t) p.n_groups * p.n_slots;
-    return p.tile_rows == 64 && p.size_k % (64 * KSLICES) == 0 && tiles <= device_cus() &&
-           (!f32 || tiles >= 32 || !dense_split_pays(p.m, p.n_slots, p.size_k));
+    if (p.tile_rows != 64 || p.size_k % (64 * KSLICES) != 0) return false;
+    const int64_t cus = device_cus() / 8, wgs = (int64_t) (p.n_groups + 7) / 8 * p.n_slots;     // of one XCD
+    const bool two_slices = f32 && dense_split_pays(p.m, p.n_slots, p.size_k);
+    if (wgs <= cus) return p.size_k >= 1024 && (!two_slices || 2 * wgs > cus);
+    return wgs <= 2 * cus && p.size_k >= 6144 && !two_slices;
 }
 
 template <int MODE>
@@ -643,7 +651,7 @@ extern "C" int exl3_linear(const uint16_t* x, int64_t m, int k, const uint16_t* 
     if (dense_kslice_pays(p, out_dtype == EXL3_DTYPE_F32))
         rc = out_dtype == EXL3_DTYPE_F32 ? launch_kslice_bits<MODE_STORE_F32>(bits, p, s)
                                          : launch_kslice_bits<MODE_STORE_F16>(bits, p, s);
-    else if (dense_kpair_pays(m, p.n_slots, k))
+    else if (p.tile_rows != 64 && dense_kpair_pays(m, p.n_slots, k))
         rc = out_dtype == EXL3_DTYPE_F32 ? launch_kpair_bits<MODE_STORE_F32>(bits, p, s)
                                          : launch_kpair_bits<MODE_STORE_F16>(bits, p, s);
     else if (out_dtype == EXL3_DTYPE_F32 && dense_split_pays(m, p.n_slots, k))
