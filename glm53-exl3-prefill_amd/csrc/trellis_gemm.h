@@ -115,8 +115,8 @@ struct GemmParams
     // SCATTER_F32 thin tiles of the decode path (trellis_gemm_actin_kernel): the fp32 gate|up sums [rows, 2 I] from
     // which each workgroup computes its own K slice of act into LDS (act_suh / act_suh_stride / act_limit as above)
     const float* act_gu;
-    // grouped 64-row tiles that read each expert's weights once (the prefill's thin launches, the decode path) load the
-    // trellis words non-temporal
+    // grouped 64- and 128-row tables that read each expert's weights once (the prefill's thin launches, the decode path)
+    // load the trellis words non-temporal
     int weights_nt;
     // a side job of the launch: clear zero[0 .. zero4) (float4s), a buffer a later launch accumulates into
     float4* zero;

@@ -1,6 +1,8 @@
 """64- and 128-row tiles (weights decoded straight into MFMA operands, activations through LDS in four-stage chunks) against the
 256-row kernel (weights decoded through LDS) bit for bit, and against the CPU oracle: row counts around every 16-row
 group, K of whole and partial chunks, every trellis width."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -92,3 +94,48 @@ def test_tail_tables(dev, tile_rows, thin_rows, T):
     for tab, e, r in ((full, fe, fr), (thin, te, tr)):
         assert list(zip(e.tolist(), r.tolist()))[:len(tab)] == tab
         assert (e[len(tab):] == -1).all()
+
+
+def kernels_of(fn):
+    """Names of the kernels `fn` launches, from a graph that captures it (nothing runs)."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        fn()
+    raw, n = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(n)) == 0
+
+    class Params(ctypes.Structure):                            # hipKernelNodeParams
+        _fields_ = [("block", ctypes.c_uint32 * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p),
+                    ("grid", ctypes.c_uint32 * 3), ("params", ctypes.c_void_p), ("shared", ctypes.c_uint32)]
+    names = []
+    for node in nodes:
+        p = Params()
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
+        names.append(hip.hipKernelNameRefByPtr(ctypes.c_void_p(p.func), None).decode())
+    return names
+
+
+@pytest.mark.parametrize("tile_rows", [64, 128])
+@pytest.mark.parametrize("mode", [0, 1, 2, 4])
+def test_weights_are_streamed_only_when_read_once(dev, tile_rows, mode):
+    """A table may hold many tiles of an expert, which share its weights through the caches: only weights_once (and not
+    with the atomic scatter) takes the kernel with non-temporal weight loads, the last template argument."""
+    E, K, N, R = 2, 128, 128, 400
+    words = torch.zeros(E, K // 16, N // 16, 64, dtype=torch.int16, device=dev)
+    half = lambda *s: torch.ones(*s, dtype=torch.float16, device=dev)  # noqa: E731
+    table = torch.zeros(4, dtype=torch.int32, device=dev)
+    out = torch.zeros(gp.t16_rows(R), N, dtype=torch.float16 if mode in (0, 4) else torch.float32, device=dev)
+    rows = torch.arange(R, dtype=torch.int32, device=dev)
+    tokens = rows.long()
+    a, svh, rw, counts = half(gp.t16_rows(R), K), half(E, N), half(R), torch.tensor([R, 0], dtype=torch.int32, device=dev)
+    for once in (False, True):
+        names = kernels_of(lambda: gp.grouped_gemm(
+            a, words, None, svh, None, table, table, counts, table[:E], tokens if mode == 1 else None,
+            rw if mode in (1, 2) else None, out if mode == 4 else out[:R], mode, route_index=rows if mode == 2 else None,
+            tile_rows=tile_rows, a_layout=1, a_rows=R, weights_once=once))
+        assert len(names) == 1 and "trellis_gemm_kernelILi4E" in names[0], names
+        assert ("Lb1EEE" in names[0]) == (once and mode != 1), names
