@@ -1486,6 +1486,7 @@ int launch_gemm_kslice(const GemmParams& p, hipStream_t s)
 template <int BITS, int MODE, bool DENSE>
 int launch_gemm(const GemmParams& p, hipStream_t s)
 {
+    if (DENSE && p.tile_rows == 128) return fail("internal: no dense kernel for 128-row tiles");
     const int groups8 = (p.n_groups + 7) / 8 * 8;
     const int64_t grid = (int64_t) groups8 * p.n_slots * (p.k_split > 1 ? p.k_split : 1);
     if (grid == 0) return EXL3_OK;

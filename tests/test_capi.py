@@ -4,6 +4,8 @@ TORCH_CHECK contract, kernel/exl3_grouped_prefill.cu:288-372, kernel/exl3_fat_ge
 import ctypes
 import os
 import re
+import shutil
+import subprocess
 
 import pytest
 import torch
@@ -405,3 +407,32 @@ def test_sort_routes_split_tiles_contract():
     for zero, n in ((None, 8), (FAKE, 6), (ctypes.c_void_p(0x1004), 8), (FAKE, -4)):
         rc, msg = call(zero=zero, n=n)
         assert rc == _lib.EXL3_ERR_ARG and "zero must be" in msg, (zero, n)
+
+
+DENSE_LAUNCH = """
+#include "trellis_gemm.h"
+using namespace exl3;
+extern "C" int dense_launch(int bits, int tile_rows)
+{
+    GemmParams p{};                                     // no row groups: nothing is launched
+    p.tile_rows = tile_rows;
+    return bits == 2 ? launch_gemm_b2(MODE_STORE_F16, true, p, nullptr)
+         : bits == 3 ? launch_gemm_b3(MODE_STORE_F16, true, p, nullptr) : launch_gemm_b4d(MODE_STORE_F16, p, nullptr);
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+def test_dense_launch_refuses_128_row_tiles(tmp_path):
+    """The dense kernels run 64-, 256- and 512-row tiles; the 64-row one would leave rows 64 .. 127 of a 128-row tile out.
+    Calls the launch inside the library from a host-only translation unit."""
+    lib = os.path.dirname(gp.library_path())
+    (tmp_path / "launch.hip").write_text(DENSE_LAUNCH)
+    subprocess.run(["hipcc", "--offload-arch=gfx950", "--offload-host-only", "-std=c++17", "-w", "-fPIC", "-shared", "-I",
+                    os.path.join(os.path.dirname(lib), "csrc"), "launch.hip", "-o", "launch.so", "-L", lib,
+                    "-lexl3_grouped", "-Wl,-rpath," + lib], cwd=tmp_path, check=True)
+    _lib.load()
+    launch = ctypes.CDLL(str(tmp_path / "launch.so")).dense_launch
+    for bits in (2, 3, 4):
+        assert [launch(bits, t) for t in (64, 256, 512)] == [_lib.EXL3_OK] * 3
+        assert launch(bits, 128) == _lib.EXL3_ERR_ARG and "128-row tiles" in _lib.last_error()
