@@ -472,9 +472,8 @@ struct Mma
     uint32_t a_off[4];
     int a_step, wread, last_kb;
 
-    // rpw: rows per wave (contiguous groups), or gstride > 0: the wave's groups are mw, mw + gstride, ...
-    __device__ __forceinline__ Mma(const GemmParams& p, const Tile& t, int mw, int lane, int num_kb, int rpw,
-                                   int gstride = 0)
+    // The wave's rows are 64 mw .. + 63, or with gstride > 0 the 16-row groups mw, mw + gstride, ...
+    __device__ __forceinline__ Mma(const GemmParams& p, const Tile& t, int mw, int lane, int num_kb, int gstride = 0)
     {
         const int tok = lane & 15, kq = lane >> 4;
         a_step = p.a_t16 ? 4 * 128 * 2 : TILE_K * 2;          // bytes per stage
@@ -486,7 +485,7 @@ struct Mma
         #pragma unroll
         for (int mb = 0; mb < 4; ++mb)
         {
-            const int row = t.row0 + min((gstride ? 16 * (mw + gstride * mb) : rpw * mw + 16 * mb) + tok,
+            const int row = t.row0 + min((gstride ? 16 * (mw + gstride * mb) : 64 * mw + 16 * mb) + tok,
                                          t.rows_valid - 1);
             a_off[mb] = p.a_t16 ? (uint32_t) ((((row >> 4) - g0) * (p.size_k >> 3) + kq) * 256 + (row & 15) * 16)
                                 : (uint32_t) ((row - t.row0) * p.size_k * 2 + 16 * kq);
@@ -953,7 +952,7 @@ __device__ __forceinline__ void thin_mainloop(const GemmParams& p, const Tile& t
     constexpr int CHUNK = TALL ? 2 : THIN_CHUNK, SLOTS = 2 * CHUNK;
     constexpr int MINE = TALL ? 2 : GROUPS, SLOT_GROUPS = TALL ? 8 : GROUPS;
     static_assert(SLOTS * SLOT_GROUPS * 1024 <= THIN_LDS_BYTES, "activation chunks");
-    const Mma mm = TALL ? Mma(p, t, wave, lane, num_kb, 64, 4) : Mma(p, t, 0, lane, num_kb, 64);
+    const Mma mm = TALL ? Mma(p, t, wave, lane, num_kb, 4) : Mma(p, t, 0, lane, num_kb);
     uint32_t raw[THIN_DEPTH][Dec::NR];
     half8_t mine[MINE];                                            // what the wave has in flight for a later chunk
     auto put = [&](int s) {                                        // TALL: stage s; else the wave's stage of chunk s / CHUNK
@@ -1134,33 +1133,33 @@ __device__ __forceinline__ void thin_tile(const GemmParams& p, const Tile& t, in
     }
 }
 
-// The main loop of a 128-, 256- or 512-row tile: the waves share each decoded stage (a barrier per stage), each
+// The main loop of a 256- or 512-row tile (four 16-row groups per wave): the waves share each decoded stage (a barrier per stage), each
 // multiplying its own rows into acc. epi (may be null): where the wave stages its epilogue inputs. Returns the number
 // of 16-row groups the wave multiplied (uniform over the wave).
-template <int BITS, int MODE, int MBN, int WAVES>
+template <int BITS, int MODE, int WAVES>
 __device__ __forceinline__ int tile_mainloop(const GemmParams& p, const Tile& t, int wave, int lane,
-                                             unsigned char* lds_raw, EpiLds* epi, floatx4 (&acc)[MBN][8])
+                                             unsigned char* lds_raw, EpiLds* epi, floatx4 (&acc)[4][8])
 {
     uint16_t* lds_b = reinterpret_cast<uint16_t*>(lds_raw);
     const int num_kb = t.num_kb;
     using Dec = typename std::conditional<WAVES == 8, Decoder1<BITS>, Decoder<BITS>>::type;
     constexpr int NR = Dec::NR;
     // 8-wave workgroups interleave the 16-row groups over the waves (wave w multiplies groups w, w + 8, ...), so a
-    // partial tile keeps both waves of every SIMD equally busy; 4-wave workgroups give each wave 16 MBN contiguous rows.
+    // partial tile keeps both waves of every SIMD equally busy; 4-wave workgroups give each wave 64 contiguous rows.
     constexpr int GSTRIDE = WAVES == 8 ? 8 : 0;
     const Dec dec(p, t, wave, lane, num_kb);
-    const Mma mm(p, t, wave, lane, num_kb, 16 * MBN, GSTRIDE);
+    const Mma mm(p, t, wave, lane, num_kb, GSTRIDE);
     const int n_groups = (t.rows_valid + 15) >> 4;
     const int n_w = GSTRIDE ? (n_groups > wave ? (n_groups - wave + GSTRIDE - 1) / GSTRIDE : 0)
-                            : min(MBN, max(0, n_groups - MBN * wave));          // this wave's groups (uniform)
+                            : min(4, max(0, n_groups - 4 * wave));          // this wave's groups (uniform)
 
     #pragma unroll
-    for (int mb = 0; mb < MBN; ++mb)
+    for (int mb = 0; mb < 4; ++mb)
         #pragma unroll
         for (int nb = 0; nb < 8; ++nb) acc[mb][nb] = {};
 
     // Main loop, specialised on the number of 16-row groups a wave multiplies (MBA: 0 = decode only, 1 for a wave with
-    // <= 16 valid rows, else MBN). Every variant runs the same barriers. Loads past the last stage are clamped to it, so
+    // <= 16 valid rows, else 4). Every variant runs the same barriers. Loads past the last stage are clamped to it, so
     // every path keeps the same loads in flight.
     // The epilogue's inputs: loaded before the pipeline's first loads, written to LDS after them (so the write waits
     // only for these), read back by the epilogue.
@@ -1170,28 +1169,26 @@ __device__ __forceinline__ int tile_mainloop(const GemmParams& p, const Tile& t,
     auto epi_load = [&]() {
         ep_svh = reinterpret_cast<const uint32_t*>(t.svh)[lane];
         if constexpr (route_mode(MODE))
-            if (lane < 16 * MBN)
-            {
-                const int mb = lane >> 4;
-                const int r_local = (GSTRIDE ? 16 * (wave + GSTRIDE * mb) : 16 * MBN * wave + 16 * mb) + (lane & 15);
-                const int64_t srow = (int64_t) t.row0 + min(r_local, t.rows_valid - 1);
-                ep_rw = h2f(p.route_weight[srow]);
-                ep_dest = (MODE == MODE_SCATTER_F32) ? p.token[srow] : (int64_t) p.route_index[srow];
-            }
+        {
+            const int mb = lane >> 4;
+            const int r_local = (GSTRIDE ? 16 * (wave + GSTRIDE * mb) : 64 * wave + 16 * mb) + (lane & 15);
+            const int64_t srow = (int64_t) t.row0 + min(r_local, t.rows_valid - 1);
+            ep_rw = h2f(p.route_weight[srow]);
+            ep_dest = (MODE == MODE_SCATTER_F32) ? p.token[srow] : (int64_t) p.route_index[srow];
+        }
     };
     auto epi_store = [&]() {
         epi->svh[lane] = ep_svh;
         if constexpr (route_mode(MODE))
-            if (lane < 16 * MBN)
-            {
-                epi->rw[lane] = ep_rw;
-                epi->dest[lane] = ep_dest;
-            }
+        {
+            epi->rw[lane] = ep_rw;
+            epi->dest[lane] = ep_dest;
+        }
     };
     auto mainloop = [&](auto mba_tag) {
         constexpr int MBA = decltype(mba_tag)::value;
         uint32_t raw[RAW_DEPTH][NR];
-        half8_t act[ACT_DEPTH][MBN];
+        half8_t act[ACT_DEPTH][4];
         {
             uint32_t r0[NR];
             if (MBA > 0 && epi) epi_load();
@@ -1240,7 +1237,6 @@ __device__ __forceinline__ int tile_mainloop(const GemmParams& p, const Tile& t,
     };
     if constexpr (GSTRIDE > 0)
     {
-        static_assert(MBN == 4, "interleaved groups: up to four per wave");
         switch (n_w)
         {
             case 4: mainloop(std::integral_constant<int, 4>{}); break;
@@ -1250,25 +1246,25 @@ __device__ __forceinline__ int tile_mainloop(const GemmParams& p, const Tile& t,
             default: mainloop(std::integral_constant<int, 0>{}); break;
         }
     }
-    else if (MBN > 1 && n_w > 1) mainloop(std::integral_constant<int, MBN>{});
+    else if (n_w > 1) mainloop(std::integral_constant<int, 4>{});
     else if (n_w > 0) mainloop(std::integral_constant<int, 1>{});
     else mainloop(std::integral_constant<int, 0>{});
     return n_w;
 }
 
-// 128-, 256- and 512-row tiles: the shared main loop, then every wave's epilogue over its rows.
-template <int BITS, int MODE, int MBN, int WAVES>
+// 256- and 512-row tiles: the shared main loop, then every wave's epilogue over its rows.
+template <int BITS, int MODE, int WAVES>
 __device__ __forceinline__ void shared_tile(const GemmParams& p, const Tile& t, int wave, int lane,
                                             unsigned char* lds_raw, EpiLds* epi)
 {
     constexpr int GSTRIDE = WAVES == 8 ? 8 : 0;
-    floatx4 acc[MBN][8];
-    const int n_w = tile_mainloop<BITS, MODE, MBN, WAVES>(p, t, wave, lane, lds_raw, epi, acc);
+    floatx4 acc[4][8];
+    const int n_w = tile_mainloop<BITS, MODE, WAVES>(p, t, wave, lane, lds_raw, epi, acc);
 
     if constexpr (atomic_mode(MODE)) __syncthreads();            // decoded tiles are dead; LDS becomes staging
     float* const stage = reinterpret_cast<float*>(lds_raw) + wave * (16 * SC_ROW);
     if (n_w == 0) return;
-    epilogue<MODE, MBN, GSTRIDE>(p, t, wave, lane, acc, stage, epi);
+    epilogue<MODE, 4, GSTRIDE>(p, t, wave, lane, acc, stage, epi);
 }
 
 // ------------------------------------------------------------------------------------------- kernel
@@ -1311,7 +1307,7 @@ void trellis_gemm_kernel(const GemmParams p)
     else
     {
         __shared__ EpiLds lds_epi[WAVES];
-        shared_tile<BITS, MODE, MBN, WAVES>(p, t, wave, lane, lds_raw, lds_epi + wave);
+        shared_tile<BITS, MODE, WAVES>(p, t, wave, lane, lds_raw, lds_epi + wave);
     }
 }
 
@@ -1375,7 +1371,7 @@ void trellis_gemm_kpair_kernel(const GemmParams p)
     th.num_kb = t.num_kb / 2;                                      // even: the host requires K % 128 == 0
     th.kb0 = t.kb0 + half * th.num_kb;
     floatx4 acc[4][8];
-    const int n_w = tile_mainloop<BITS, MODE, 4, 4>(p, th, wave, lane, lds_raw + half * LDS_MAIN_BYTES,
+    const int n_w = tile_mainloop<BITS, MODE, 4>(p, th, wave, lane, lds_raw + half * LDS_MAIN_BYTES,
                                                     half ? nullptr : lds_epi + wave, acc);
     floatx4* xs = reinterpret_cast<floatx4*>(lds_raw) + wave * 8 * 64 + lane;
     #pragma unroll
