@@ -271,6 +271,54 @@ def test_split_gemm_contract():
     assert rc == _lib.EXL3_ERR_ARG and "2I" in msg
 
 
+def test_tail_tiles_contract():
+    need = _lib.load().exl3_sort_routes_workspace_bytes(100, 8, 288)
+    args = dict(ids=FAKE, ids_dt=_lib.DTYPE_I64, w=FAKE, w_dt=_lib.DTYPE_F32, T=100, k=8, E=288, ts=FAKE, ws=FAKE, eor=FAKE,
+                ri=None, counts=FAKE, row0=FAKE, work=FAKE, bytes=need, tile_rows=256, thin_rows=128, mf=12, mt=288,
+                fe=FAKE, fr=FAKE, te=FAKE, tr=FAKE, meta=FAKE, zero=None, n=0)
+
+    def call(entry="exl3_sort_routes_tail_tiles", **kw):
+        a = dict(args)
+        a.update(kw)
+        return rc_and_msg(entry, *a.values(), None)
+
+    for kw, text in ((dict(thin_rows=96), "thin_rows 64 or 128"), (dict(thin_rows=256), "thin_rows 64 or 128"),
+                     (dict(tile_rows=64), "tile_rows must be"), (dict(E=1025), "too many experts"),
+                     (dict(bytes=need - 1), "workspace"), (dict(meta=None), "null pointer"), (dict(fr=None), "null pointer"),
+                     (dict(zero=FAKE, n=6), "zero"), (dict(ids_dt=_lib.DTYPE_F32), "int64 or int32"), (dict(mf=-1), "table")):
+        rc, msg = call(**kw)
+        assert rc == _lib.EXL3_ERR_ARG and text in msg, (kw, msg)
+    rc, msg = call("exl3_sort_routes_split_tiles")                       # its second table keeps 64 rows
+    assert rc == _lib.EXL3_ERR_ARG and msg.endswith("thin_rows 64")
+
+
+def test_weights_once_contract():
+    args = dict(a=FAKE, a_rows=256, size_k=512, a_layout=1, pg=FAKE, pu=None, es=32 * 16 * 64, tk=32, tn=16, bits=4, sg=FAKE,
+                su=None, ss=256, be=FAKE, br=FAKE, mb=10, tile_rows=128, counts=FAKE, row0=FAKE, E=8, tok=FAKE, rw=FAKE,
+                ri=None, out=FAKE, out_rows=256, mode=1, k_split=1, zero=None, n=0)
+    for kw, text in ((dict(tile_rows=256), "64 or 128"), (dict(tile_rows=512), "64 or 128"), (dict(bits=5), "bits"),
+                     (dict(size_k=500), "K mismatch"), (dict(mode=5), "mode must be"), (dict(mode=0, k_split=2), "accumulating"),
+                     (dict(zero=FAKE, n=6), "zero must be"), (dict(be=None), "null pointer")):
+        a = dict(args)
+        a.update(kw)
+        rc, msg = rc_and_msg("exl3_grouped_gemm_once", *a.values(), None)
+        assert rc == _lib.EXL3_ERR_ARG and text in msg, (kw, msg)
+
+
+def test_row_had_gather_bf16_contract():
+    args = dict(src=FAKE, dst=FAKE, tok=FAKE, eor=FAKE, suh=FAKE, stride=256, len=256, rows=4, K=256)
+    odd = ctypes.c_void_p(0x1002)
+    for kw, text in ((dict(K=100, len=100), "multiple of 128"), (dict(len=128), "match suh"), (dict(rows=-1), "row count"),
+                     (dict(src=odd), "aligned"), (dict(dst=odd), "aligned"), (dict(stride=252), "aligned"),
+                     (dict(src=None), "null pointer"), (dict(tok=None), "null pointer"), (dict(eor=None), "null pointer")):
+        a = dict(args)
+        a.update(kw)
+        rc, msg = rc_and_msg("exl3_row_had_gather_bf16", *a.values(), None)
+        assert rc == _lib.EXL3_ERR_ARG and text in msg, (kw, msg)
+    args.update(src=None, rows=0)
+    assert rc_and_msg("exl3_row_had_gather_bf16", *args.values(), None)[0] == _lib.EXL3_OK
+
+
 DECODE_ARGS = dict(x=FAKE, tokens=4, hidden=4096, ids=FAKE, ids_dt=4, w=FAKE, w_dt=0, topk=8, E=288, inter=768,
                    bits=4, pg=FAKE, pu=FAKE, es13=2 * 256 * 48 * 64, suh=FAKE, suh_s=8192, svg=FAKE, svu=FAKE,
                    sv_s=1536, pd=FAKE, es2=48 * 256 * 64, suhd=FAKE, suhd_s=768, svd=FAKE, svd_s=4096,
@@ -307,6 +355,25 @@ def test_moe_decode_contract():
     assert rc == _lib.EXL3_ERR_ARG and "workspace too small" in msg
     rc, msg = decode_call(tokens=0, x=None, ids=None, w=None, out=None, ws=None)
     assert rc == _lib.EXL3_OK                            # nothing to do: no pointer is needed
+
+
+def test_moe_decode_dt_contract():
+    need = _lib.load().exl3_moe_decode_workspace_bytes(4, 8, 288, 4096, 768)
+
+    def call(x_dtype=_lib.DTYPE_BF16, **kw):
+        a = dict(DECODE_ARGS)
+        a.update(kw)
+        a = list(a.values())
+        return rc_and_msg("exl3_moe_decode_dt", a[0], x_dtype, *a[1:], None)
+
+    for kw, text in ((dict(x_dtype=_lib.DTYPE_F32), "fp16 or bf16"), (dict(x_dtype=_lib.DTYPE_I64), "fp16 or bf16"),
+                     (dict(x=None), "null pointer"), (dict(hidden=4000), "multiples of 128"),
+                     (dict(ws_bytes=need - 1), "workspace too small"),
+                     (dict(x=ctypes.c_void_p(0x1002), ws_bytes=need), "aligned"),
+                     (dict(x=ctypes.c_void_p(0x1002), ws_bytes=need, x_dtype=_lib.DTYPE_F16), "aligned")):
+        rc, msg = call(**kw)
+        assert rc == _lib.EXL3_ERR_ARG and text in msg, (kw, msg)
+    assert call(tokens=0, x=None, ids=None, w=None, out=None, ws=None)[0] == _lib.EXL3_OK
 
 
 def test_moe_decode_noalloc_contract():

@@ -42,8 +42,13 @@ def test_layer_bf16_matches_cast(dev, T, shift):
     b = rt.grouped_prefill(x.to(torch.float16), ids, w, TL, 10.0, scatter="combine")
     assert torch.equal(a.view(torch.int32), b.view(torch.int32))
     layer = (TL.w13_trellis, TL.w13_suh, TL.w13_svh, TL.w2_trellis, TL.w2_suh, TL.w2_svh)
+    rt._decode_ws.clear()                                       # sized by this test
+    got = [rt.moe_decode(x, ids, w, TL, 10.0)]                  # shift 1: cast in front
     if shift == 0:
-        c, d = gp.moe_decode_dt(x, ids, w, *layer, 10.0), gp.moe_decode(x.to(torch.float16), ids, w, *layer, 10.0)
+        got.append(gp.moe_decode_dt(x, ids, w, *layer, 10.0))
+    rt._decode_ws.clear()                                       # later tests size their own
+    d = gp.moe_decode(x.to(torch.float16), ids, w, *layer, 10.0)
+    for c in got:
         # the same launches add fp32 partial sums in an order of their own: a few 2^-24 per sum, and an fp16 step of a
         # gate|up value where that crosses a rounding boundary
         assert (c - d).norm() <= 1e-4 * d.norm()

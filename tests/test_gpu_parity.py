@@ -184,12 +184,15 @@ def test_build_tiles_split_bit_exact(dev, kind, T, E, k, tile_rows):
     assert (fe[len(full):] == -1).all() and (te[len(thin):] == -1).all()
 
 
-def fused_prep(ids_t, w_t, E, tile_rows, fused, zero_n=0):
-    """The prefill preparation as sort_routes + build_tiles_split (fused=False) or as sort_routes_split_tiles: every
-    output, from buffers pre-filled with sentinels."""
+def fused_prep(ids_t, w_t, E, tile_rows, fused, zero_n=0, tail_rows=None):
+    """The route preparation as sort_routes + build_tiles_split (fused=False) or as sort_routes_split_tiles, or with
+    tail_rows as sort_routes_tail_tiles (what the prefill runs) at its smallest table: every output, from buffers
+    pre-filled with sentinels."""
     dev = ids_t.device
     R = ids_t.numel()
     mf, mt = R // tile_rows + E, min(E, R)
+    if tail_rows:
+        mf = min(mf, max(1, R // min(tile_rows, 65)))
     out = dict(ts=torch.full((R,), -3, dtype=torch.int64, device=dev),
                ws=torch.full((R,), 7.0, dtype=torch.float16, device=dev),
                eor=torch.full((R,), -3, dtype=torch.int32, device=dev),
@@ -204,7 +207,11 @@ def fused_prep(ids_t, w_t, E, tile_rows, fused, zero_n=0):
                zero=torch.full((zero_n + 8,), float("nan"), dtype=torch.float32, device=dev))
     o = out
     z = o["zero"][4:-4] if zero_n else None
-    if fused:
+    if tail_rows:
+        work = gp.sort_routes_tail_tiles(ids_t, w_t, E, o["ts"], o["ws"], o["eor"], o["counts"], o["row0"], o["fe"],
+                                         o["fr"], o["te"], o["tr"], o["meta"], tile_rows, tail_rows, zero=z,
+                                         route_index=o["ri"])
+    elif fused:
         work = gp.sort_routes_split_tiles(ids_t, w_t, E, o["ts"], o["ws"], o["eor"], o["counts"], o["row0"], o["fe"],
                                           o["fr"], o["te"], o["tr"], o["meta"], tile_rows, 64, zero=z,
                                           route_index=o["ri"])
@@ -224,8 +231,7 @@ SPLIT_TILE_CASES = ([r + (256,) for r in ROUTINGS] +
 
 @pytest.mark.parametrize("kind,T,E,k,tile_rows", SPLIT_TILE_CASES)
 def test_sort_routes_split_tiles_matches_two_ops(dev, kind, T, E, k, tile_rows):
-    """The prefill path's two-launch preparation (histogram; scatter with per-workgroup cursors + tile tables +
-    output clear) writes exactly what sort_routes followed by build_tiles_split writes (kernel/exl3_grouped_runtime.py
+    """The two-launch preparation (histogram; scatter with per-workgroup cursors + tile tables + output clear) writes exactly what sort_routes followed by build_tiles_split writes (kernel/exl3_grouped_runtime.py
     :59-68, kernel/exl3_grouped_prefill.cu:63-96), bit for bit, with int64 and int32 ids; the clear covers exactly the
     given range."""
     ids, w = synth.make_routing(kind, T, E, k, seed=T + 9)
@@ -260,6 +266,38 @@ def test_sort_routes_split_tiles_empty_and_dropped(dev):
     assert b["dropped"] == int((ids < 0).sum() + (ids >= 40).sum()) > 0
     for n in a:
         assert np.array_equal(np.atleast_1d(a[n]).view(np.uint8), np.atleast_1d(b[n]).view(np.uint8)), n
+
+
+def dropped_ids(T, E, k):
+    rng = np.random.default_rng(T + E)
+    ids = rng.integers(0, E, (T, k)).astype(np.int64)
+    ids[::7, k - 1] = -1
+    ids[5::11, 0] = E
+    return ids, rng.random((T, k)).astype(np.float32)
+
+
+@pytest.mark.parametrize("tail_rows", [64, 128])
+@pytest.mark.parametrize("kind,T,E,k,tile_rows", SPLIT_TILE_CASES + [("dropped", 3000, 41, 8, 256), ("dropped", 700, 24, 6, 128),
+                                                                     ("dropped", 0, 16, 8, 256)])
+def test_sort_routes_tail_tiles_every_output(dev, kind, T, E, k, tile_rows, tail_rows):
+    """The prefill's preparation: the sorted routes, counts, clear and dropped count of sort_routes_split_tiles bit for bit,
+    and the two tables of the closed form, whose limit is 128 rows only where last tiles of 65 to 128 rows number more
+    than half the larger ones; int64 and int32 ids, experts in and out of whole groups of four, dropped ids, no routes."""
+    ids, w = dropped_ids(T, E, k) if kind == "dropped" else synth.make_routing(kind, T, E, k, seed=T + 9)
+    counts = np.bincount(ids[(ids >= 0) & (ids < E)], minlength=E)
+    rem = counts % tile_rows
+    limit = 128 if tail_rows == 128 and 2 * ((rem > 64) & (rem <= 128)).sum() > (counts // tile_rows + (rem > 128)).sum() else 64
+    full, thin, rows = split_tables(counts, tile_rows, min(limit, tile_rows - 1))
+    wt = torch.from_numpy(w).to(dev)
+    for ids_dt in (torch.int64, torch.int32):
+        it = torch.from_numpy(ids).to(ids_dt).to(dev)
+        a = fused_prep(it, wt, E, tile_rows, fused=True, zero_n=T * 4 * 5)
+        b = fused_prep(it, wt, E, tile_rows, fused=True, zero_n=T * 4 * 5, tail_rows=tail_rows)
+        for n in ("ts", "ws", "eor", "counts", "row0", "ri", "zero", "dropped"):
+            assert np.array_equal(np.atleast_1d(a[n]).view(np.uint8), np.atleast_1d(b[n]).view(np.uint8)), n
+        assert b["meta"].tolist() == [len(full), rows, len(thin)]
+        for tab, e, r in ((full, b["fe"], b["fr"]), (thin, b["te"], b["tr"])):
+            assert list(zip(e[:len(tab)].tolist(), r[:len(tab)].tolist())) == tab and (e[len(tab):] == -1).all()
 
 
 def test_prefill_thin_tiles_match_one_table(dev):
