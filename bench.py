@@ -44,6 +44,7 @@ MFMA_F16_PEAK_TFLOPS = 2500.0      # MI355X dense fp16 (no sparsity)
 # I=1024 per rank, routing_skewed(hot=12, share=0.55), real checkpoint layer 3): reference README.md:41-44.
 REFERENCE_GB10_MS = {1024: 11.4, 2048: 13.7, 4096: 20.2, 8192: 33.2}
 HBM_PEAK_GBS = 8000.0
+PEAK_CLOCK_MHZ = 2400
 # The kernels of each stage of grouped_prefill as rocprofv3 names them (namespaces and parameter lists stripped; the keys
 # of the committed profile summaries): the GEMMs run full expert tiles on the main kernel and each expert's last tile
 # of at most 64 (128 where such tiles are many) rows on the thin one.
@@ -169,12 +170,14 @@ def traffic_from_profiles(workload: str, kernels):
 def mfma_busy_from_profiles(workload: str, kernels):
     """Matrix-pipe busy fraction of a stage's launches from the committed SQ counter summary: sum of
     SQ_VALU_MFMA_BUSY_CYCLES over the launches / (their GRBM_GUI_ACTIVE cycles per XCD x SIMDs), and the shader clock
-    the same counters imply; None if missing."""
+    the same counters imply; None if missing. GRBM_GUI_ACTIVE runs a little longer than the launch: a launch counts no
+    more cycles than its time holds at the peak clock."""
     j = profile_json(f"grouped_prefill_{workload}_sq_counters")
     try:
         ks = [j["kernels"][k] for k in kernels]
         busy = sum(k["SQ_VALU_MFMA_BUSY_CYCLES"] for k in ks)
-        cycles = sum(k["GRBM_GUI_ACTIVE"] / j["xcds"] for k in ks)
+        cycles = sum(min(j["kernels"][k]["GRBM_GUI_ACTIVE"] / j["xcds"], j["launch_us"][k] * PEAK_CLOCK_MHZ)
+                     for k in kernels)
         return {"mfma_busy": round(busy / (cycles * j["simds"]), 4),
                 "valu_busy": round(sum(k["SQ_ACTIVE_INST_VALU"] for k in ks) * 4 / (cycles * j["simds"]), 4),
                 "clock_mhz": j.get("clock_mhz", {}).get(kernels[0])}

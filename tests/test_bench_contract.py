@@ -48,3 +48,13 @@ def test_stage_kernels_are_in_the_kernel_trace(bench):
     for st, ks in stage_kernels(bench, "combine").items():
         for k in ks:
             assert k in kernels, (st, k)
+
+
+def test_counted_cycles_stay_within_the_launch(bench, monkeypatch):
+    """A launch whose counted cycles imply more than the peak clock is priced by its time at that clock."""
+    k = {"SQ_VALU_MFMA_BUSY_CYCLES": 24000.0, "SQ_ACTIVE_INST_VALU": 12000.0}
+    j = {"xcds": 8, "simds": 10, "clock_mhz": {"a": 2000, "b": 4000}, "launch_us": {"a": 10.0, "b": 10.0},
+         "kernels": {"a": dict(k, GRBM_GUI_ACTIVE=8 * 20000.0), "b": dict(k, GRBM_GUI_ACTIVE=8 * 40000.0)}}
+    monkeypatch.setattr(bench, "profile_json", lambda name: j)
+    assert bench.mfma_busy_from_profiles("any", ["a"]) == {"mfma_busy": 0.12, "valu_busy": 0.24, "clock_mhz": 2000}
+    assert bench.mfma_busy_from_profiles("any", ["b"])["valu_busy"] == 0.2
