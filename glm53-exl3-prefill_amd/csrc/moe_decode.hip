@@ -4,8 +4,8 @@
 //
 // Same stages and rounding points as the grouped prefill -- route sort, gather + input Hadamard, gate|up GEMM,
 // activation + Hadamard, down GEMM with scatter -- on a fixed launch sequence whose grids depend on the sizes only:
-//   * 64-row tiles on the thin GEMM kernel (16 rows per wave, a quarter of the accumulators, four workgroups per CU):
-//     most waves of a small batch only decode, and the extra resident waves hide the trellis loads' latency.
+//   * 64-row tiles on the thin GEMM kernel (each wave decodes its own 32 columns for all row groups of the tile; four
+//     workgroups per CU): a small batch is decode work, and the extra resident waves hide the trellis loads' latency.
 //   * The row-tile table is bounded by min(E, R) + R / 64 entries (every expert with rows adds at most one partial
 //     tile), so a batch of a few tokens launches a few dozen row tiles instead of one per expert.
 //   * A batch of a few tokens has too few (row tile, column tile) pairs to fill the GPU, so both GEMMs split K into
@@ -29,7 +29,7 @@ static __device__ __align__(256) unsigned char scratch[DECODE_SCRATCH_BYTES];
 namespace exl3 {
 namespace {
 
-constexpr int DECODE_TILE_ROWS = 64;                 // the thin GEMM kernel: 16 rows per wave, four workgroups per CU
+constexpr int DECODE_TILE_ROWS = 64;                 // the thin GEMM kernel: four workgroups per CU
 constexpr int SMALL_ROUTES = 2048;                   // routes exl3_route_prep_small sorts in one workgroup
 
 __global__ __launch_bounds__(256)
@@ -119,19 +119,20 @@ int k_split_for(int64_t wgs, int stages, int target)
     return best;
 }
 
+// Whether the gate|up launch and the down launch with the activation pass inside load the trellis words
+// non-temporal (each call reads each active expert's weights once). Per call in a step's graph, non-temporal / cached
+// us at 4 bits: one token 22.6 / 24.1, 2 tokens 36.1 / 37.4, 3 49.4 / 49.7, 4 58.5 / 57.4, 6 89.9 / 90.4, 8 100.8 /
+// 101.5, 16 172 / 174, 32 250 / 258, 64 359 / 362, 128 424 / 428 (2 and 3 bits: even to 6% faster non-temporal at every
+// size). The limits were drawn on an earlier 64-row kernel, where 2 and 4 tokens lost 3 us; what is left between them is
+// within 4%. The down launch after a separate activation pass (more than 16 routes) lost with them there at every size.
+bool decode_weights_nt(int64_t routes) { return routes <= 8 || routes >= 64; }
+
 // K slices for the down launch with the activation pass inside (trellis_gemm_actin_kernel): equal slices of whole
 // 128-column act blocks, at most ACTIN_MAX_KB stages each, with the cost rule of k_split_for but the fewest
 // workgroups among equals (at one token 2 slices of 12 stages ran 30.3-30.5 us per call in a step's graph, 3 slices
 // of 8 stages 30.6-30.8: each slice adds its partial rows into the same output row, and the act work per slice is
 // spread over the waves either way); 0 when no such split fits one round of `target` workgroups (the gate|up launch
 // then keeps the pass).
-// Whether the gate|up launch and the down launch with the activation pass inside load the trellis words
-// non-temporal (each call reads each active expert's weights once). Measured per call in a step's graph (two
-// alternating runs): one token 25.6-26.0 vs 26.7-26.8 us, 16 tokens 172-177 vs 183-184, 32 tokens 262-266 vs 276-277,
-// 64 tokens 400 vs 403-405; at 2 and 4 tokens the non-temporal loads measured 2.8-3 us slower, at 8 and 128 even. The
-// down launch after a separate activation pass (more than 16 routes) measured slower with them at every size.
-bool decode_weights_nt(int64_t routes) { return routes <= 8 || routes >= 64; }
-
 int k_split_actin(int64_t wgs, int stages, int target)
 {
     if (wgs <= 0 || stages % 4 != 0) return 0;

@@ -4,8 +4,8 @@
 // Workgroup = 4 waves, tile = up to 256 rows x 128 output columns (one H128 block), K stage = 32.
 //   * Each stage's 16 trellis tiles (32 x 128 weights) are decoded ONCE per workgroup -- a 16-lane row per tile, every
 //     lane decoding two 8-weight chunks from one coalesced load of its own stream words -- into a k-contiguous [n][k]
-//     fp16 tile in LDS, and reused by all four waves for every row of the tile. A row tile covers `tile_rows` (128 or
-//     256) rows of one expert, so each decoded weight feeds up to 256 rows of MFMA work.
+//     fp16 tile in LDS, and reused by all four waves for every row of the tile. A row tile covers up to 256 rows of one
+//     expert, so each decoded weight feeds up to 256 rows of MFMA work.
 //   * Each wave owns 64 rows x 128 columns and runs v_mfma_f32_16x16x32_f16 with the DECODED WEIGHTS as the first
 //     operand and the activations as the second (out^T in the accumulators: a lane owns one row and 32 columns). The
 //     activation operand of one MFMA is 16 rows x 64 contiguous bytes, so each activation load instruction touches 16
@@ -24,8 +24,8 @@
 //   * Activations and trellis words are read through buffer resources: fixed per-lane offsets plus a scalar stage
 //     offset, and zero instead of a fault outside the operand.
 // Variants of the same kernel: 8 waves (512-row tiles, one workgroup per CU, each wave decoding one chunk per lane) for
-// 512-row tiles and large dense GEMMs. 64-row tiles (small batches, each expert's small last tile) run a kernel of their
-// own (thin_tile): four workgroups per CU, each wave decoding its own 32 columns straight into MFMA operands.
+// 512-row tiles and large dense GEMMs. 64- and 128-row tiles (small batches, each expert's small last tile) run a kernel
+// of their own (thin_tile): four workgroups per CU, each wave decoding its own 32 columns straight into MFMA operands.
 #pragma once
 #include "exl3_common.h"
 #include "hadamard.h"
@@ -93,7 +93,7 @@ struct GemmParams
     const int32_t* block_row0;
     const int32_t* counts;
     const int32_t* expert_row0;
-    int tile_rows;                 // rows per row tile (grouped: 128, 256 or 512; dense: 64 x waves)
+    int tile_rows;                 // rows per row tile (64, 256 or 512; grouped also 128)
     int n_groups;                  // row tiles (grouped: table entries; dense: ceil(m / tile_rows))
     int n_slots;                   // 128-col tiles over all tensors
     int n_tiles_each;              // 128-col tiles per tensor
@@ -933,9 +933,10 @@ __device__ __forceinline__ void act_store(const GemmParams& p, const Tile& t, in
 // over. (Every wave loading all row groups itself moves four times the bytes out of L2, which then bounds the launch: 451
 // against 348 us below. Decoding each stage once per workgroup through LDS, as the taller tiles do, makes every wave read
 // the whole 8 KB stage for one row group: at four workgroups per CU that is 96 KB per stage, 770 of ~1900 cycles.)
-// Bound: VALU issue of the decode, 70 instructions per wave and stage, at the clock the power limit leaves (1.6-1.9 GHz
-// in these launches); 8 trellis stages in flight or five workgroups per CU measured the same. 288 experts x ~28 rows, K =
-// 4096, N = 1536: 392 -> 348 us; K = 768, N = 4096 with the atomic scatter 235 -> 214 us. Afterwards the accumulators go
+// Bound: VALU issue of the decode, 70 instructions per wave and stage, at the clock the power limit leaves; 8 trellis
+// stages in flight or five workgroups per CU measured the same. 288 experts x ~28 rows, K = 4096, N = 1536: 392 -> 348
+// us (in a counter run, each launch by itself, 303 us at 2.15 GHz with the VALU 87% busy: the same cycles in 348 us are
+// 1.87 GHz); K = 768, N = 4096 with the atomic scatter 235 -> 214 us. Afterwards the accumulators go
 // through LDS so that wave g holds row group g over all 128 columns, the layout of the shared epilogue.
 // ACT_IN (one row group): the activation operand is computed by the workgroup itself (act_load / act_store around the
 // first trellis loads) and read from LDS instead of loaded.
@@ -1268,7 +1269,7 @@ __device__ __forceinline__ void shared_tile(const GemmParams& p, const Tile& t, 
 }
 
 // ------------------------------------------------------------------------------------------- kernel
-// 128- and 256-row tiles: every wave decodes a quarter of each stage and multiplies its own 64 rows; two workgroups
+// 256-row tiles: every wave decodes a quarter of each stage and multiplies its own 64 rows; two workgroups
 // share a CU. Pipeline of stage s: barrier; read stage s's weight fragments; decode stage s+1 while stage s's MFMAs run;
 // write stage s+1 into the other of two LDS buffers; issue loads for later stages.
 template <int WAVES> constexpr int lds_scatter_bytes() { return WAVES * 16 * SC_ROW * 4; }
@@ -1407,7 +1408,8 @@ int launch_gemm_kpair(const GemmParams& p, hipStream_t s)
 }
 
 // A dense GEMM of so few rows that its 64-row tiles leave CUs idle (a small decode batch's projection: 32 workgroups for 4096
-// columns) lasts as long as one workgroup's whole K range: latency, at one wave per SIMD. Here one workgroup of 16 waves
+// columns, one on each CU of the one XCD that a row group's tiles run on) lasts as long as one workgroup's whole K range:
+// latency, at one wave per SIMD. Here one workgroup of 16 waves
 // takes the tile, KSLICES groups of four waves over equal parts of K, each the thin main loop with its own activation
 // chunks (the barriers are shared: all run the same stages); the partial sums are then added through LDS in slice order,
 // so the result is the same on every run, and the first group's waves run the epilogue. A linear of 7 x 4096 x 4096 with

@@ -468,9 +468,11 @@ int fat_common(const uint16_t* a, int64_t m, int size_k, const uint16_t* packed,
 
 // Single-expert row tiles. A single expert's matrix is short next to the device: 256-row tiles of a 2048 x 4096 x 4096
 // GEMM are 256 workgroups for 256 CUs. 64-row tiles on the thin kernel (four workgroups per CU) decode each weight
-// once per 64 rows instead of 256 but spread the work over four times the workgroups, which wins up to 256 rows, and
-// up to 2048 rows when K is short (K < 2048: fewer stages to decode per tile). Larger matrices take 512-row tiles on
-// the 8-wave kernel. Measured per call (gate|up M x 4096 x 2048, down M x 1024 x 4096, M = 128 .. 2048).
+// once per 64 rows instead of 256 but spread the work over four times the workgroups: up to 256 rows, and up to 2048
+// rows when K is short (K < 2048: fewer stages to decode per tile). Larger matrices take 512-row tiles on the 8-wave
+// kernel. The limits were drawn on an earlier 64-row kernel; on the present one the linear's fp16 output would gain from
+// 64-row tiles up to about 1024 rows (64 / 512 rows per tile: 512 x 4096 x 4096 40 / 105 us, 1024 x 4096 x 4096 74 / 105,
+// 1024 x 4096 x 2048 41 / 102) and from 256-row tiles around 2048 rows of a short K (2048 x 768 x 4096: 27.5 against 33.1).
 int dense_tile_rows(int64_t m, int size_k)
 {
     if (m <= 256 || (m <= 2048 && size_k < 2048)) return 64;
@@ -558,8 +560,9 @@ template <int MODE>
 int launch_dense_split2(GemmParams p, int bits, float* out, int64_t out_floats, hipStream_t s, int variant = 1)
 {
     const int total_kb = p.size_k / TILE_K;
-    // thin tiles here too, up to 1024 rows (measured); a fixed-schedule variant keeps its tiles (at most 256 rows:
-    // the slices add with the 4-wave kernels)
+    // thin tiles here too, up to 1024 rows (64 / 256 rows per tile: 512 x 4096 x 2048 31 / 45 us, 1024 x 4096 x 2048 45 /
+    // 50, 2048 x 4096 x 2048 73 / 66); a fixed-schedule variant keeps its tiles (at most 256 rows: the slices add with the
+    // 4-wave kernels)
     p.tile_rows = variant == 1 ? (p.m <= 1024 ? 64 : 256) : std::min(p.tile_rows, 256);
     p.n_groups = (int) ((p.m + p.tile_rows - 1) / p.tile_rows);
     p.kb_per_split = ((total_kb + 1) / 2 + 1) / 2 * 2;        // even: both slices have an even number of stages
