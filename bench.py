@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the EXL3 grouped routed-expert MoE prefill on one MI355X.
 
-Workload (BASELINE.json configs[3], the shape the metric is quoted on): one TP rank's share of a 288-expert layer,
+Workload (the shape the metric is quoted on): one TP rank's share of a 288-expert layer,
 H=4096, I=768, 4 bpw trellis, an 8192-token chunk, top-8 routing skewed by a Zipf(1.1) prior; synthetic seeded
 inputs resident in HBM before timing starts. A step is one full grouped_prefill call (route sort, block table,
 gather + input Hadamard, gate|up GEMM, SwiGLU + down Hadamard, down GEMM and its output by token: at this size the
@@ -22,9 +22,9 @@ reference's prototype loop: dequantised fp16 weights, per-expert matmuls, index_
 the active experts, dequant and loop timed apart and extrapolated to the layer.
 
   python bench.py [--steps K] [--warmup W] [--tokens T] [--bits B] [--routing R] [--no-cpu-baseline]
-  python bench.py --sweep          (extra lines for T = 1024, 2048, 4096, 8192; not the driver's contract line)
+  python bench.py --sweep          (extra lines for T = 1024, 2048, 4096, 8192; not the benchmark line)
   python bench.py --decode         (the decode path, moe_decode, at small batches of the same layer: one line per
-                                    batch, eager and graph-replayed; not the driver's contract line)
+                                    batch, eager and graph-replayed; not the benchmark line)
   python bench.py --fat            (the per-expert fat GEMM per call: config 2 and the reference's published shapes)
   python bench.py --config repro --tokens T   (the reference's published grouped-path shape; vs_baseline = its GB10
                                     per-layer ms / this run's)

@@ -1,4 +1,4 @@
-"""Seeded synthetic inputs for the five BASELINE.json configs (numpy on the host; see to_device()).
+"""Seeded synthetic inputs for five workloads (numpy on the host; see to_device()).
 
 A layer is one TP rank's share of a routed-expert MoE: trellis codes are uniform random 16-bit words,
 suh are +-1 sign vectors (gate and up share theirs, as kernel/test_grouped.py:82-84 requires), svh are
@@ -15,15 +15,15 @@ from dataclasses import dataclass, field
 import numpy as np
 
 CONFIGS = {
-    # BASELINE.json configs[0]: tiny layer, CPU-runnable
+    # tiny layer, CPU-runnable
     "tiny": dict(E=8, H=512, I=256, bits=4, T=128, topk=2, routing="softmax"),
-    # configs[1]: single-expert fat GEMM (exl3_fat_gemm drop-in), gate|up concatenated
+    # single-expert fat GEMM (exl3_fat_gemm drop-in), gate|up concatenated
     "fat": dict(M=4096, K=4096, N=1536, bits=4),
-    # configs[2]: full 288-expert layer, 1024-token chunk
+    # full 288-expert layer, 1024-token chunk
     "layer1k": dict(E=288, H=4096, I=768, bits=4, T=1024, topk=8, routing="softmax"),
-    # configs[3]: headline, 8192 tokens, Zipf(1.1)-skewed top-8 (sweep 1K/2K/4K/8K)
+    # headline, 8192 tokens, Zipf(1.1)-skewed top-8 (sweep 1K/2K/4K/8K)
     "headline": dict(E=288, H=4096, I=768, bits=4, T=8192, topk=8, routing="zipf", zipf_s=1.1),
-    # configs[4]: thin-expert stress at 4 bpw (repeated at 3 and 2 bpw)
+    # thin-expert stress at 4 bpw (repeated at 3 and 2 bpw)
     "thin": dict(E=288, H=4096, I=768, bits=4, T=7168, topk=8, routing="thin"),
     # the shape of the reference's own published grouped-path numbers (README.md:41-44: I = 1024 per rank,
     # routing_skewed(hot=12, share=0.55), T = 1K / 2K / 4K / 8K), with synthetic codes in place of the checkpoint

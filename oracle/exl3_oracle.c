@@ -1,7 +1,7 @@
 /*
  * exl3_oracle.c -- CPU restatement of the integer / bit-level half of the EXL3 grouped MoE prefill path.
  *
- * TEST INFRASTRUCTURE ONLY. This file is the checker the parity tests, __graft_entry__.smoke() and the
+ * TEST INFRASTRUCTURE ONLY. This file is the oracle the parity tests, __graft_entry__.smoke() and the
  * bench's cpu_baseline leg compare the HIP kernels against. Nothing in the product path links, loads or
  * calls it; the product fails loudly when its HIP library is missing.
  *

@@ -1,7 +1,7 @@
 """CPU oracle for the EXL3 grouped routed-expert MoE prefill path.
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg, and
-there only as the checker (or the timed CPU baseline). The product path never imports it.
+there only as the oracle (or the timed CPU baseline). The product path never imports it.
 
 Two layers:
   * exl3_oracle.c (via ctypes): bit-level trellis decode, route sort, block table, fp16 rounding.

@@ -2,10 +2,10 @@
 """Writes the golden fixtures under tests/golden/ from this repo's own CPU oracle and generators.
 
 The reference ships no vectors, KATs or fixtures for this path (its tests need exllamav3, the vLLM overlay, a
-real checkpoint and CUDA), so these fixtures pin the GPU <-> oracle relation and the generators across
-rounds, not the oracle <-> exllamav3 relation (that stays "parity unpinned").
+real checkpoint and CUDA), so these fixtures pin the GPU <-> oracle relation and the generators over
+time, not the oracle <-> exllamav3 relation (that stays "parity unpinned").
 
-  tiny.npz      config 1: sha256 of every generated input, the routing, sort and
+  tiny.npz      the tiny workload: sha256 of every generated input, the routing, sort and
                 block-table outputs (bit-exact), the stage outputs h13 / gu / act (fp16) and the layer output
                 of both the staged oracle and the expert loop (fp32).
   decode.json   sha256 of the 65536-entry decode table, a 1024-entry sample, and decoded tiles of a fixed

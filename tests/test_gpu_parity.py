@@ -1,7 +1,7 @@
 """GPU parity: the HIP kernels (through the C ABI) against the CPU oracle on the same seeded inputs.
 
 Bars: bit-exact for integer / byte work (decode, reconstruct, route sort, block table); for floating point the
-north-star tolerance rel L2 <= 1e-3 against the oracle (tighter bars are asserted where the arithmetic allows:
+required rel L2 <= 1e-3 against the oracle (tighter bars are asserted where the arithmetic allows:
 fp16 stage outputs may differ from the float64 oracle by one fp16 rounding step, fp32 GEMM outputs by fp32
 accumulation order). At the headline size, where the full CPU loop is too slow for a test, parity is checked on
 sampled tokens plus size-independent properties (linearity in the route weights, token-permutation
@@ -866,7 +866,7 @@ def test_headline_sampled_tokens_and_properties(dev, scatter):
 @pytest.mark.parametrize("scatter", [None, "atomic"])
 @pytest.mark.parametrize("T", [1024, 2048, 4096])
 def test_headline_routing_sweep_sampled_tokens(dev, T, scatter):
-    """The headline layer and Zipf routing at the sweep's smaller chunks (BASELINE.json configs[3]), sampled tokens
+    """The headline layer and Zipf routing at the sweep's smaller chunks, sampled tokens
     against the expert loop, through the shipped output method (None: "auto", the combine from 16384 routes) and the
     atomic scatter."""
     L, x, ids, w, cfg = synth.make_config("headline", seed=0, T=T)
@@ -881,8 +881,8 @@ def test_full_output_vs_expert_loop(dev, name, T, bits):
     """Every token of the output through the shipped output method (scatter None: "auto") against the expert loop,
     as the reference checks its grouped path (kernel/test_grouped.py:148-155: the whole output at 256 and 2048 tokens,
     skewed routing, which the repro config restates): the headline layer and Zipf routing at 2048 tokens and at the
-    full 8192-token chunk (BASELINE.json configs[3]), the reference's own shape (I = 1024, skewed routing), and the
-    headline layer with 3- and 2-bit trellis codes (configs[4] repeats the hot path at those widths)."""
+    full 8192-token chunk, the reference's own shape (I = 1024, skewed routing), and the
+    headline layer with 3- and 2-bit trellis codes."""
     L, x, ids, w, cfg = synth.make_config(name, seed=0, T=T, bits=bits)
     out = run_layer(L, x, ids, w, dev).cpu().numpy()
     ref = O.expert_loop(x, ids, w, to_np_layer(L), LIMIT)

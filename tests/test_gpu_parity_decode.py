@@ -2,7 +2,7 @@
 where the reference calls the overlay's fused exl3_moe) and its building blocks, the split-K grouped GEMM and the
 fp32-input act_had.
 
-Bars: the north-star rel L2 <= 1e-3 against the oracle expert loop (harness/proto_fp8.py:123-134 restated in
+Bars: the required rel L2 <= 1e-3 against the oracle expert loop (harness/proto_fp8.py:123-134 restated in
 oracle/exl3_oracle.py); exact equality where the arithmetic is the same (fp32 act_had input rounded to fp16, a
 one-slice mode-3 GEMM against the fp16 store); fp32 accumulation-order bounds where only the order of additions
 differs (K slices, atomics). Graph capture: replays with fresh inputs against eager calls.

@@ -1,4 +1,4 @@
-"""Pins the CPU oracle (oracle/exl3_oracle.{c,py}) before it is trusted as the checker.
+"""Pins the CPU oracle (oracle/exl3_oracle.{c,py}) before it is trusted.
 
 Every check compares the oracle with something it did not compute itself: numpy / scipy library routines,
 closed forms worked by hand, brute force over the abstract definition, or invariants a plausible slip
@@ -288,7 +288,7 @@ def test_gemm_stage_commutes_with_real_domain_weight():
 
 @pytest.mark.parametrize("bits", [4, 3, 2])
 def test_linear_is_x_times_real_domain_weight(bits):
-    """The dense linear equals x @ diag(suh) H W' H diag(svh) up to the fp16 rounding of h."""
+    """The dense linear equals x @ diag(suh) H W' H diag(svh) up to the fp16 rounding of h (rel L2 <= 1e-3)."""
     rng = np.random.default_rng(bits)
     K, N, M = 256, 384, 24
     x = rng.standard_normal((M, K)).astype(np.float16)

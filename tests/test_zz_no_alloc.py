@@ -1,6 +1,6 @@
 """GPU test of exl3_moe_decode_noalloc, the decode entry point that allocates nothing (its workspace is the library's
 fixed per-GPU scratch array): called through the C ABI, its output must equal exl3_moe_decode's (the same kernels on a
-caller workspace) up to the fp32 atomic summation order, and meet the north-star rel L2 <= 1e-3 against the oracle
+caller workspace) up to the fp32 atomic summation order, and meet the required rel L2 <= 1e-3 against the oracle
 expert loop -- on two calls in a row, the second with fewer tokens (the scratch keeps the first call's contents)."""
 import ctypes
 
