@@ -746,11 +746,11 @@ def test_fat_gemm_short_k(dev, M, K, bits):
 
 @pytest.mark.parametrize("bits", [4, 3, 2])
 def test_thin_tile_epilogues_bit_identical(dev, bits):
-    """Thin tiles of at most 16 rows (the column-split loop, its results gathered in LDS for wave 0's epilogue; one-row
-    tiles in the fp32 atomic modes take a one-row epilogue, two columns per lane) must give the shared loop's outputs
-    bit for bit. Dense calls of 1, 2, 5 and 16 rows (thin tiles) against the same rows of a 20-row call (the shared
-    loop), for the fp32 store (K = 1024), the K-split fp32 atomic store (K = 4096: two slices added onto zero) and the
-    routed scatter (one add per token), and against the oracle."""
+    """Thin tiles (64-row tables and short matrices: the column-split loop, its results gathered in LDS for the epilogue;
+    one-row tiles in the fp32 atomic modes take a one-row epilogue, two columns per lane) must give the shared loop's
+    outputs bit for bit. Dense calls of 1, 2, 5, 16 and 20 rows (thin tiles of one and two row groups) against the same
+    rows of a 20-row call on 256-row tiles (the shared loop), for the fp32 store (K = 1024), the K-split fp32 atomic store
+    (K = 4096: two slices added onto zero) and the routed scatter (one add per token), and against the oracle."""
     M = 20
     tok = np.random.default_rng(bits).permutation(40)[:M].astype(np.int64)
     rw = (np.random.default_rng(bits + 1).random(M) * 0.5 + 0.25).astype(np.float16)
@@ -758,25 +758,26 @@ def test_thin_tile_epilogues_bit_identical(dev, bits):
         a, packed, svh = synth.make_fat(7 + K, M=M, K=K, N=256, bits=bits)
         ref = O.fat_gemm(a, packed, svh, dtype=np.float32)
         outs, scat = {}, {}
-        for m in (1, 2, 5, 16, M):
-            out = torch.full((m, 256), float("nan"), dtype=torch.float32, device=dev)
-            gp.fat_gemm_v2(t16(a[:m], dev), t16(packed, dev), out, t16(svh, dev), bits, True, False, 1)
+        for m, variant in ((1, 1), (2, 1), (5, 1), (16, 1), (M, 1), ("shared", 2)):
+            n = M if m == "shared" else m
+            out = torch.full((n, 256), float("nan"), dtype=torch.float32, device=dev)
+            gp.fat_gemm_v2(t16(a[:n], dev), t16(packed, dev), out, t16(svh, dev), bits, True, False, variant)
             outs[m] = out.cpu().numpy()
             sc = torch.zeros(40, 256, dtype=torch.float32, device=dev)
-            gp.fat_gemm_v2_scatter(t16(a[:m], dev), t16(packed, dev), sc, t16(svh, dev), t16(tok[:m], dev),
-                                   t16(rw[:m], dev), bits, True, False, 1)
+            gp.fat_gemm_v2_scatter(t16(a[:n], dev), t16(packed, dev), sc, t16(svh, dev), t16(tok[:n], dev),
+                                   t16(rw[:n], dev), bits, True, False, variant)
             scat[m] = sc.cpu().numpy()
-        assert O.rel_l2(outs[M], ref) < 1e-5
-        assert O.rel_l2(scat[M][tok], ref * rw[:, None].astype(np.float32)) < 1e-5
-        for m in (1, 2, 5, 16):
-            assert np.array_equal(outs[m].view(np.uint32), outs[M][:m].view(np.uint32)), (K, m)
-            assert np.array_equal(scat[m][tok[:m]].view(np.uint32), scat[M][tok[:m]].view(np.uint32)), (K, m)
+        shared = outs["shared"], scat["shared"]
+        assert O.rel_l2(shared[0], ref) < 1e-5
+        assert O.rel_l2(shared[1][tok], ref * rw[:, None].astype(np.float32)) < 1e-5
+        for m in (1, 2, 5, 16, M):
+            assert np.array_equal(outs[m].view(np.uint32), shared[0][:m].view(np.uint32)), (K, m)
+            assert np.array_equal(scat[m][tok[:m]].view(np.uint32), shared[1][tok[:m]].view(np.uint32)), (K, m)
             assert not np.delete(scat[m], tok[:m], axis=0).any()
 
 
 def test_thin_tile_epilogue_grouped_bit_identical(dev):
-    """The grouped GEMM's thin tiles (64-row tables: the thin kernel, experts of 1-16 rows on the column-split loop)
-    against the same rows on 256-row tiles (the shared loop): the fp16 gate|up rows and the down projection's per-route
+    """The grouped GEMM's thin tiles (64-row tables) against the same rows on 256-row tiles (the shared loop): the fp16 gate|up rows and the down projection's per-route
     fp32 rows bit for bit, at the headline routing over 256 tokens."""
     L, x, ids, w, cfg = synth.make_config("headline", seed=4, T=256)
     E, H, I = cfg["E"], cfg["H"], cfg["I"]

@@ -249,7 +249,7 @@ def sorted_case(cfg, T, seed, dev, tile_rows=128, routing="softmax"):
 @pytest.mark.parametrize("tile_rows", [64, 128, 256])
 @pytest.mark.parametrize("T", [1, 16, 300])
 def test_split_gate_up_matches_store(dev, T, tile_rows):
-    """Mode 3 (64-row tiles: the thin kernel) against the fp16 store of mode 0 on a 128-row table."""
+    """Mode 3 (64- and 128-row tiles: the thin kernel) against the fp16 store of mode 0 on a 128-row table."""
     L, cfg = layer_case("layer1k")
     TL = device_layer("layer1k")
     x, ids, w, (ts, ws, eor, counts, row0), be, br = sorted_case(cfg, T, 11, dev, tile_rows)
